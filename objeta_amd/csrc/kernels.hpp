@@ -142,4 +142,30 @@ int32_t launch_moe_grouped(objeta_hip_context* ctx, int32_t format, hipStream_t 
                            const float* x, const float* resid, float* out, uint64_t hidden, uint64_t inter,
                            uint64_t out_dim, float limit);
 
+// The same layer for many tokens (wide.hip): work items of up to 32 tokens of an
+// expert, any number of tokens (in slices of 4096 assignments). Against the sets of 8
+// (hidden 2048, intermediate 768, top-8, Q4_0, us per layer): 24 tokens 75 / 71, 48
+// tokens 89 / 104.
+constexpr uint64_t kWideMinTokens = 32;
+bool wide_supported(int32_t format, uint64_t n_table, uint64_t n_tokens, uint64_t k, uint64_t hidden, uint64_t inter,
+                    uint64_t out_dim);
+int32_t launch_moe_wide(objeta_hip_context* ctx, int32_t format, hipStream_t s, const objeta_hip_expert_ptrs* table,
+                        uint64_t n_table, const objeta_hip_expert_ptrs* shared, const uint32_t* ids, const float* wts,
+                        uint64_t n_tokens, uint64_t k, const float* x, const float* resid, float* out, uint64_t hidden,
+                        uint64_t inter, uint64_t out_dim, float limit);
+// The batched GEMV from kGemvWideMinBatch vectors (wide.hip; where gemv_mfma_kernel
+// would take a second pass); shapes and alignment as gemv_mfma_supported. Q4_0, us
+// against the passes: 9 vectors by 2048 x 2048 14.2 / 15.2, 16 by 14336 x 4096 26.5 /
+// 35.4, 128 84 / 275.
+constexpr uint64_t kGemvWideMinBatch = 9;
+bool gemv_wide_supported(int32_t format, uint64_t rows, uint64_t cols, uint64_t batch);
+int32_t launch_gemv_wide(objeta_hip_context* ctx, hipStream_t s, int32_t format, const void* w, const void* ws,
+                         const float* x, float* y, uint64_t rows, uint64_t cols, uint64_t batch);
+// out = resid + sum_j w_j part_j (+ shared part), and the sum of a GEMV's column ranges.
+void launch_moe_combine(hipStream_t s, const uint32_t* ids, const float* wts, const float* part,
+                        const float* shared_part, const float* resid, float* out, uint32_t n_tokens, uint32_t k,
+                        uint32_t out_dim, uint32_t n_table);
+void launch_gemv_reduce(hipStream_t s, const float* part, float* y, uint32_t rows, uint32_t n_vec, uint32_t n_ranges);
+
+
 }  // namespace objeta
