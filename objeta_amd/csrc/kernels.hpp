@@ -84,7 +84,7 @@ int32_t launch_moe_official_fp4(objeta_hip_context* ctx, hipStream_t s, const ob
                                 uint64_t hidden, uint64_t inter, uint64_t out_dim, float limit,
                                 uint8_t* inter_values, uint8_t* inter_scales, const OfficialMarks* marks);
 
-// The same layer on the grouped-token products (grouped.hip), for batches of at
+// The same layer on the grouped-token products (wide.hip), for batches of at
 // least kOfficialGroupedMinTokens tokens in the grouped path's limits (at the
 // DeepSeek shape the per-token kernels are faster up to 4 tokens, the grouped ones
 // from 6: the per-token path reads the FP8 shared expert once per token).
@@ -142,11 +142,11 @@ int32_t launch_moe_grouped(objeta_hip_context* ctx, int32_t format, hipStream_t 
                            const float* x, const float* resid, float* out, uint64_t hidden, uint64_t inter,
                            uint64_t out_dim, float limit);
 
-// The same layer for many tokens (wide.hip): work items of up to 32 tokens of an
-// expert, any number of tokens (in slices of 4096 assignments). Against the sets of 8
-// (hidden 2048, intermediate 768, top-8, Q4_0, us per layer): 24 tokens 75 / 71, 48
-// tokens 89 / 104.
-constexpr uint64_t kWideMinTokens = 32;
+// The same layer on the wide products (wide.hip): work items of up to 16 or 32 tokens of
+// an expert, any number of tokens. Split FP4 takes them at any batch, the block formats
+// from 9 tokens (below, sets of 8 hold every expert's tokens: Q5_0 3072 x 2048 at 3 tokens
+// 57 us on them, 66 here; Q4_0 2048 x 768 at 16 tokens 60 / 57, at 48 104 / 83).
+constexpr uint64_t kWideMinTokens = 9;
 bool wide_supported(int32_t format, uint64_t n_table, uint64_t n_tokens, uint64_t k, uint64_t hidden, uint64_t inter,
                     uint64_t out_dim);
 int32_t launch_moe_wide(objeta_hip_context* ctx, int32_t format, hipStream_t s, const objeta_hip_expert_ptrs* table,

@@ -37,7 +37,7 @@ __device__ __forceinline__ int split_shift(float m) {
 // lo = fp16(x 2^s - hi), stored in the (w0,w4),(w1,w5),.. order of each group of
 // 8 when perm is set, else in element order; mult[row] = 2^-s restores the
 // products. s comes from the finite elements; an infinity or NaN is its own hi part
-// (lo 0), so it propagates as in a plain product.
+// (lo 0), so it propagates as in a plain product. lo may be NULL (hi alone).
 __device__ inline void split_row(const float* __restrict__ src, uint32_t cols, _Float16* __restrict__ hi,
                           _Float16* __restrict__ lo, float* __restrict__ mult, uint32_t row, uint32_t perm) {
     __shared__ float red[4];
@@ -68,7 +68,7 @@ __device__ inline void split_row(const float* __restrict__ src, uint32_t cols, _
             vl[d] = __builtin_isfinite(xs) ? static_cast<_Float16>(xs - static_cast<float>(th)) : static_cast<_Float16>(0.0f);
         }
         *reinterpret_cast<half8*>(h + 8 * g) = vh;
-        *reinterpret_cast<half8*>(l + 8 * g) = vl;
+        if (lo) *reinterpret_cast<half8*>(l + 8 * g) = vl;
     }
 }
 
@@ -120,15 +120,12 @@ __device__ __forceinline__ half8 iq3_to_b(uint32_t lo16, uint32_t h8) {
 }
 
 // ------------------------------------------------------------- staged tiles
-// Staged row segments of a 16-row slab: weights (and, for the split FP4 layout,
-// the E8M0 scales) of columns [c0, c0 + kc), row stride padded by one dword so the
-// lanes of different rows read different banks. kChunkGU / kChunkDn: columns per
-// staged chunk for gate and up together / for down (16 and 8 blocks of 32 for the
-// block formats, 16 and 16 for split FP4: the widths that measured fastest, as
-// narrower chunks keep more workgroups resident; 8 blocks of FP8 bytes fill the
-// same LDS). kTileScale: one
-// E8M0 byte per 128 x 128 tile (FP8), taken per chunk into a register by
-// tile_scales instead of being staged per row.
+// Staged row segments: weights (and, for the split FP4 layout, the E8M0 scales) of columns
+// [c0, c0 + kc). wdw / sdw: dwords of a row segment. kChunkGU / kChunkDn (block formats):
+// columns per staged chunk of the eight-member sets (grouped.hip), gate and up together /
+// down, the widths that measured fastest there. kTileScale: one E8M0 byte per 128 x 128
+// tile (FP8), taken per chunk into a register by tile_scales instead of being staged per
+// row.
 template <class R>
 struct Tile;
 
@@ -170,12 +167,8 @@ struct Tile<Fp4Rows> {
     static constexpr bool kPermuted = false;
     static constexpr bool kScales = true;
     static constexpr bool kTileScale = false;
-    static constexpr uint32_t kChunkGU = 512, kChunkDn = 512;
     static constexpr __host__ __device__ uint32_t wdw(uint32_t kc) { return kc / 8; }   // kc / 2 bytes
     static constexpr __host__ __device__ uint32_t sdw(uint32_t kc) { return kc / 128; }  // kc / 32 bytes (kc % 128 == 0)
-    static constexpr __host__ __device__ uint32_t lds_dw(uint32_t kc) {
-        return kSlab * (wdw(kc) + 4) + kSlab * (sdw(kc) + 1);
-    }
     static __device__ __forceinline__ size_t wpitch(const Fp4Rows& m) { return m.wrow; }
     static __device__ __forceinline__ size_t spitch(const Fp4Rows& m) { return m.srow; }
     static __device__ __forceinline__ const uint8_t* wrow(const Fp4Rows& m, uint32_t c0) { return m.w + c0 / 2; }
@@ -202,10 +195,8 @@ struct Tile<Fp8Rows> {
     static constexpr bool kPermuted = false;
     static constexpr bool kScales = false;
     static constexpr bool kTileScale = true;
-    static constexpr uint32_t kChunkGU = 256, kChunkDn = 256;
     static constexpr __host__ __device__ uint32_t wdw(uint32_t kc) { return kc / 4; }  // kc bytes
     static constexpr __host__ __device__ uint32_t sdw(uint32_t) { return 0; }
-    static constexpr __host__ __device__ uint32_t lds_dw(uint32_t kc) { return kSlab * (wdw(kc) + 4); }
     static __device__ __forceinline__ size_t wpitch(const Fp8Rows& m) { return m.wrow; }
     static __device__ __forceinline__ size_t spitch(const Fp8Rows&) { return 0; }
     static __device__ __forceinline__ const uint8_t* wrow(const Fp8Rows& m, uint32_t c0) { return m.w + c0; }

@@ -39,45 +39,50 @@ using namespace dev;
 
 constexpr uint32_t kWMaxTable = 1024;   // experts per table
 constexpr uint32_t kWMaxAssign = 4096;  // assignments (tokens * k) per launch
-// Vector tiles of 16 per work item (two tiles and the parts' sums apart do not fit 168
-// registers: split FP4 at three sums and two tiles spilled 80 to 92 bytes).
-template <class R>
-constexpr int kWTiles = 2;
-template <>
-constexpr int kWTiles<Fp4Rows> = 1;
-template <class R>
-constexpr uint32_t kWMembersOf = 16u * kWTiles<R>;
-constexpr uint32_t kWChunk = 128;       // columns per staged chunk
-constexpr uint32_t kFlush = 2;          // chunks per running sum
-constexpr uint32_t kWRows = 128;        // weight rows per workgroup, over all matrices
-constexpr uint32_t kWAStride = kWChunk + 8;  // halves per staged vector part: 68 dwords, so the
-                                             // 16 rows of an operand read start 4 banks apart
 
-// One work item: up to 64 assignments that selected the same expert, their act rows
-// order[first .. first + count).
+// The shape of a workgroup's work: MT vector tiles of 16 per work item, RT row tiles of
+// 16 per wave (32 RT weight rows per workgroup, over all matrices), CH columns per staged
+// chunk, W waves per SIMD, the parts of the vectors (1: the low parts are zero).
+template <int MT, int RT, uint32_t CH, int W, int PARTS = 2>
+struct Work {
+    static constexpr int kMT = MT, kRT = RT, kWaves = W, kParts = PARTS;
+    static constexpr uint32_t kMembers = 16 * MT, kRows = 32 * RT, kChunk = CH;
+};
+// Large matrices at many vectors; small ones or few vectors (more workgroups, longer
+// chunks); large split FP4 ones (whose sums of the two parts stay apart, which takes the
+// registers of a second vector tile: three sums and two tiles spilled 80 to 92 bytes);
+// the official layer's, whose vectors have no low part.
+using WorkLarge = Work<2, 4, 128, 3>;
+using WorkSmall = Work<1, 2, 256, 4>;
+using WorkLarge4 = Work<1, 4, 256, 4>;
+using WorkOfficial = Work<1, 4, 256, 4, 1>;
+using WorkOfficialSmall = Work<1, 2, 256, 4, 1>;
+
+// One work item: assignments that selected the same expert, its table entry copied in and
+// their act rows (past count: the last one), so a workgroup reaches its weights and
+// vectors through one load.
 struct WideSet {
     objeta_hip_expert_ptrs p;
-    uint32_t first, count, pad[2];
+    uint32_t count, pad[3];
+    uint16_t row[32];
 };
-static_assert(sizeof(WideSet) == 64, "one 64-byte record per set");
-
-struct WideWs {
-    uint32_t* hdr;    // [0] number of sets
-    WideSet* sets;
-    uint2* order;     // {act row, token} grouped by expert, then the shared expert's
-};
+static_assert(sizeof(WideSet) == 128, "one line per set");
 
 // Groups the assignments by expert (workgroup of 256). An assignment's place among its
 // expert's comes from an LDS atomic, so the order inside an expert is not fixed; it
 // decides only which lane multiplies a row, not the row's arithmetic.
+// The shared expert (when given) follows as one more group of `shared_members` per set:
+// member t is token t, its act row n_assign + t; its sets go to shared_sets, their number
+// to hdr[1] (hdr[0]: the routed sets), or after the routed ones when shared_sets is NULL.
 __device__ void group_wide(const uint32_t* __restrict__ ids, uint32_t n_assign, uint32_t n_table,
                            const objeta_hip_expert_ptrs* __restrict__ table,
-                           const objeta_hip_expert_ptrs* __restrict__ shared, uint32_t n_tokens, WideWs w,
-                           uint32_t k, uint32_t members, uint32_t* __restrict__ err) {
+                           const objeta_hip_expert_ptrs* __restrict__ shared, uint32_t n_tokens, uint32_t members,
+                           uint32_t* __restrict__ hdr, WideSet* __restrict__ sets, WideSet* __restrict__ shared_sets,
+                           uint32_t* __restrict__ err) {
     __shared__ uint32_t cnt[kWMaxTable];
-    __shared__ uint32_t pos[kWMaxTable];
+    __shared__ uint16_t first[kWMaxTable];  // the expert's first set
     __shared__ uint16_t rank[kWMaxAssign];
-    __shared__ uint32_t wtot[2][4];
+    __shared__ uint32_t wtot[4];
     const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     for (uint32_t e = tid; e < n_table; e += 256) cnt[e] = 0;
     __syncthreads();
@@ -90,82 +95,70 @@ __device__ void group_wide(const uint32_t* __restrict__ ids, uint32_t n_assign, 
     }
     if (bad) atomicOr(err, 1u);
     __syncthreads();
-    // exclusive prefixes over experts of the counts and of the sets; thread t owns
-    // experts [t*per, (t+1)*per)
+    // exclusive prefix over experts of the sets; thread t owns experts [t*per, (t+1)*per)
     const uint32_t per = (n_table + 255) / 256;
     const uint32_t e0 = tid * per < n_table ? tid * per : n_table;
     const uint32_t e1 = e0 + per < n_table ? e0 + per : n_table;
-    uint32_t sc = 0, ss = 0;
-    for (uint32_t e = e0; e < e1; ++e) {
-        sc += cnt[e];
-        ss += (cnt[e] + members - 1) / members;
-    }
-    uint32_t ic = sc, is = ss;
+    uint32_t ss = 0;
+    for (uint32_t e = e0; e < e1; ++e) ss += (cnt[e] + members - 1) / members;
+    uint32_t is = ss;
 #pragma unroll
     for (int off = 1; off < 64; off <<= 1) {
-        const uint32_t oc = __shfl_up(ic, off, 64), os = __shfl_up(is, off, 64);
-        if (static_cast<int>(lane) >= off) {
-            ic += oc;
-            is += os;
-        }
+        const uint32_t os = __shfl_up(is, off, 64);
+        if (static_cast<int>(lane) >= off) is += os;
     }
-    if (lane == 63) {
-        wtot[0][wave] = ic;
-        wtot[1][wave] = is;
-    }
+    if (lane == 63) wtot[wave] = is;
     __syncthreads();
-    uint32_t bc = 0, bs = 0, tc = 0, ts = 0;
+    uint32_t ps = is - ss, ts = 0;
     for (uint32_t v = 0; v < 4; ++v) {
-        if (v < wave) {
-            bc += wtot[0][v];
-            bs += wtot[1][v];
-        }
-        tc += wtot[0][v];
-        ts += wtot[1][v];
+        if (v < wave) ps += wtot[v];
+        ts += wtot[v];
     }
-    uint32_t pc = bc + ic - sc, ps = bs + is - ss;
     for (uint32_t e = e0; e < e1; ++e) {
-        pos[e] = pc;
+        first[e] = static_cast<uint16_t>(ps);
         for (uint32_t j = 0; j < cnt[e]; j += members) {
-            WideSet* dst = &w.sets[ps++];
+            WideSet* dst = &sets[ps++];
             dst->p = table[e];
-            dst->first = pc + j;
             dst->count = cnt[e] - j < members ? cnt[e] - j : members;
         }
-        pc += cnt[e];
     }
-    if (shared) {
-        const uint32_t n_sh = (n_tokens + members - 1) / members;
-        for (uint32_t s = tid; s < n_sh; s += 256) {
-            const uint32_t t0 = s * members;
-            WideSet* dst = &w.sets[ts + s];
+    const uint32_t n_sh = shared ? (n_tokens + members - 1) / members : 0;
+    WideSet* const sh = shared_sets ? shared_sets : sets + ts;
+    for (uint32_t i = tid; i < n_sh * members; i += 256) {
+        const uint32_t t = i < n_tokens ? i : n_tokens - 1;
+        WideSet* dst = &sh[i / members];
+        dst->row[i % members] = static_cast<uint16_t>(n_assign + t);
+        if (i % members == 0) {
             dst->p = *shared;
-            dst->first = tc + t0;
-            dst->count = n_tokens - t0 < members ? n_tokens - t0 : members;
+            dst->count = n_tokens - i < members ? n_tokens - i : members;
         }
-        for (uint32_t t = tid; t < n_tokens; t += 256) w.order[tc + t] = make_uint2(n_assign + t, t);
-        ts += n_sh;
     }
-    if (tid == 0) w.hdr[0] = ts;
+    if (tid == 0) {
+        hdr[0] = shared_sets ? ts : ts + n_sh;
+        hdr[1] = n_sh;
+    }
     __syncthreads();
 #pragma unroll 4
     for (uint32_t a = tid; a < n_assign; a += 256) {
         const uint32_t e = ids[a];
-        if (e < n_table) w.order[pos[e] + rank[a]] = make_uint2(a, a / k);
+        if (e >= n_table) continue;
+        const uint32_t r = rank[a];
+        WideSet* dst = &sets[first[e] + r / members];
+        dst->row[r % members] = static_cast<uint16_t>(a);
+        if (r + 1 == cnt[e])  // the last one fills the rest of its set
+            for (uint32_t q = r % members + 1; q < members; ++q) dst->row[q] = static_cast<uint16_t>(a);
     }
 }
 
 // Block 0 groups the assignments; block 1 + t splits row t of x.
-__global__ __launch_bounds__(256) void wide_prepare_kernel(const uint32_t* __restrict__ ids, uint32_t n_assign,
-                                                           uint32_t n_table,
-                                                           const objeta_hip_expert_ptrs* __restrict__ table,
-                                                           const objeta_hip_expert_ptrs* __restrict__ shared,
-                                                           uint32_t n_tokens, uint32_t k, uint32_t members, WideWs w,
-                                                           uint32_t* __restrict__ err,
-                                                           const float* __restrict__ x, uint32_t cols,
-                                                           _Float16* __restrict__ xh, _Float16* __restrict__ xl,
-                                                           float* __restrict__ xmult, uint32_t perm) {
-    if (blockIdx.x == 0) group_wide(ids, n_assign, n_table, table, shared, n_tokens, w, k, members, err);
+__global__ __launch_bounds__(256) void wide_prepare_kernel(
+    const uint32_t* __restrict__ ids, uint32_t n_assign, uint32_t n_table,
+    const objeta_hip_expert_ptrs* __restrict__ table, const objeta_hip_expert_ptrs* __restrict__ shared,
+    uint32_t n_tokens, uint32_t members, uint32_t* __restrict__ hdr, WideSet* __restrict__ sets,
+    WideSet* __restrict__ shared_sets, uint32_t* __restrict__ err, const float* __restrict__ x, uint32_t cols,
+    _Float16* __restrict__ xh, _Float16* __restrict__ xl, float* __restrict__ xmult, uint32_t perm) {
+    if (blockIdx.x == 0)
+        group_wide(ids, n_assign, n_table, table, shared, n_tokens, members, hdr, sets, shared_sets, err);
     else split_row(x, cols, xh, xl, xmult, blockIdx.x - 1, perm);
 }
 
@@ -179,87 +172,112 @@ __global__ __launch_bounds__(256) void wide_split_kernel(const float* __restrict
 enum WideMode { kWGateUp = 0, kWDown = 1, kWGemv = 2 };
 
 // LDS of a workgroup: the weight rows (kStride dwords each; an odd multiple of 4, so 16
-// rows spread over all banks), the FP4 scale dwords, then both parts of the vectors.
-template <class R>
+// rows spread over all banks), the FP4 scale dwords, then both parts of the vectors
+// (rows padded by 8 halves: 4 dwords past a multiple of 64, so the 16 rows of an operand
+// read start 4 banks apart).
+template <class R, class K>
 struct WideLds {
-    static constexpr uint32_t kSeg = Tile<R>::wdw(kWChunk);  // weight dwords per row and chunk
+    static constexpr uint32_t kSeg = Tile<R>::wdw(K::kChunk);  // weight dwords per row and chunk
     static constexpr uint32_t kStride = ((kSeg + 3) / 4 | 1u) * 4;
-    static constexpr uint32_t kW = kWRows * kStride;
-    static constexpr uint32_t kS = Tile<R>::kScales ? kWRows : 0u;
-    static constexpr uint32_t kA = kWMembersOf<R> * kWAStride;  // dwords of both parts
+    static constexpr uint32_t kSdw = Tile<R>::kScales ? Tile<R>::sdw(K::kChunk) : 0u;
+    static constexpr uint32_t kAStride = K::kChunk + 8;  // halves per staged vector part
+    static constexpr uint32_t kW = K::kRows * kStride;
+    static constexpr uint32_t kS = K::kRows * kSdw;
+    static constexpr uint32_t kA = K::kMembers * kAStride * K::kParts / 2;  // dwords
     static constexpr uint32_t kDwords = kW + kS + kA;
+    // the other column half's sums: 2 row halves x RT x MT tiles x 64 lanes x 16 bytes
+    static_assert(kDwords >= 2u * K::kRT * K::kMT * 64 * 4, "the sums fit the staging LDS");
 };
-static_assert(WideLds<QRows<kQ5>>::kStride == 28 && WideLds<QRows<kQ4>>::kStride == 20, "odd multiples of 4");
-// the other half's sums (2 row halves x 4 row tiles x 4 vector tiles x 64 lanes x 16 bytes)
-static_assert(WideLds<QRows<kIQ3>>::kDwords >= 2 * 4 * kWTiles<QRows<kIQ3>> * 64 * 4, "the sums fit the staging LDS");
 
 // MODE kWGateUp: rows = inter over the split x rows, writes act; kWDown: rows = out_dim
 // over the split act rows, writes part; kWGemv: one matrix (w0, s0), vector group
 // blockIdx.z, column range blockIdx.y of `range` columns, writes out[range][vec][row].
 // The MoE modes take a linear grid: workgroup b runs on XCD b % 8 and takes row block
 // (b / 8) % nrb of set b % 8 + 8 * (b / (8 nrb)), so all row blocks of a set read its
-// vectors through one L2; sets past the device's count leave at once. FULL: every chunk is whole (else the last has 64 columns).
-template <class R, int MODE, bool FULL>
-__global__ __launch_bounds__(256, 3) void wide_products_kernel(
-    WideWs gw, const void* __restrict__ w0, const void* __restrict__ s0, const _Float16* __restrict__ vh,
-    const _Float16* __restrict__ vl, const float* __restrict__ vmult, float* __restrict__ out, uint32_t cols,
-    uint32_t rows, uint32_t n_vec, uint32_t range, uint32_t nrb, float limit,
-    uint32_t official) {
-    constexpr int kMT = kWTiles<R>;
-    constexpr uint32_t kWMembers = kWMembersOf<R>;
-    using L = WideLds<R>;
+// vectors through one L2; sets past the device's count leave at once. FULL: every chunk is whole.
+struct WideArgs {
+    const uint32_t* n;     // number of sets (MoE modes)
+    const WideSet* sets;
+    const void *w0, *s0;   // the matrix (kWGemv)
+    const _Float16 *vh, *vl;
+    const float* vmult;
+    float* out;
+    uint32_t cols, rows, k_inv, n_assign, n_vec, range, nrb;
+    float limit;
+    uint32_t official;
+};
+
+template <class R, class K, int MODE, bool FULL>
+__device__ __forceinline__ void wide_body(const WideArgs& g, const uint32_t* __restrict__ set_count,
+                                          const WideSet* __restrict__ sets, uint32_t wg) {
+    using L = WideLds<R, K>;
     using TR = Tile<R>;
+    constexpr int kMT = K::kMT, kRT = K::kRT, kParts = K::kParts;
+    constexpr uint32_t kMembers = K::kMembers, kChunk = K::kChunk;
     constexpr int kMats = MODE == kWGateUp ? 2 : 1;
-    constexpr bool kApart = TR::kScales;  // the parts' sums apart
-    constexpr uint32_t kMatRows = kWRows / kMats;
+    constexpr bool kApart = TR::kScales && kParts == 2;  // the parts' sums apart
+    constexpr uint32_t kFlush = (TR::kScales || kParts == 1 ? 8 : 4) * 64 / kChunk;  // chunks per running sum
+    constexpr uint32_t kMatRows = K::kRows / kMats;
     constexpr uint32_t kUpr = (L::kSeg + 3) / 4;                // 16-byte units per row
     constexpr uint32_t kNU = (kMatRows * kUpr + 255) / 256;      // units per thread and matrix
+    constexpr uint32_t kAUpr = kChunk / 8;                       // 16-byte units of a vector part
+    constexpr uint32_t kAStep = 256 / kAUpr;                     // vectors per round of units
+    constexpr uint32_t kNA = kMembers / kAStep;                  // rounds
+    const uint32_t cols = g.cols, rows = g.rows, n_assign = g.n_assign, n_vec = g.n_vec, nrb = g.nrb;
+    const _Float16* __restrict__ const vh = g.vh;
+    const _Float16* __restrict__ const vl = g.vl;
     extern __shared__ __align__(16) uint32_t wl[];
     uint32_t* const sl = wl + L::kW;
-    _Float16* const al = reinterpret_cast<_Float16*>(wl + L::kW + L::kS);  // [part][member][kWAStride]
+    _Float16* const al = reinterpret_cast<_Float16*>(wl + L::kW + L::kS);  // [part][member][L::kAStride]
     const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const uint32_t wr = wave & 1, wk = wave >> 1;
     const uint32_t n16 = lane & 15, kg = lane >> 4;
-    __shared__ uint32_t s_row[kWMembers];  // the members' act rows
-    __shared__ float s_mul[kWMembers];     // and the powers of two of their split vectors
-    uint32_t rb, first, m, c_begin, c_end;
+    __shared__ uint32_t s_row[kMembers];  // the members' act rows
+    __shared__ float s_mul[kMembers];     // and the powers of two of their split vectors
+    uint32_t rb, m, c_begin, c_end, first = 0;
     const void *pw[kMats], *ps[kMats];
+    const WideSet* S = nullptr;
     if constexpr (MODE == kWGemv) {
         rb = blockIdx.x;
-        c_begin = blockIdx.y * range;
-        c_end = c_begin + range < cols ? c_begin + range : cols;
-        first = blockIdx.z * kWMembers;
-        m = n_vec - first < kWMembers ? n_vec - first : kWMembers;
-        pw[0] = w0;
-        ps[0] = s0;
+        c_begin = blockIdx.y * g.range;
+        c_end = c_begin + g.range < cols ? c_begin + g.range : cols;
+        first = blockIdx.z * kMembers;
+        m = n_vec - first < kMembers ? n_vec - first : kMembers;
+        pw[0] = g.w0;
+        ps[0] = g.s0;
     } else {
-        const uint32_t b = blockIdx.x, j = b >> 3;
+        const uint32_t b = wg, j = b >> 3;
         rb = j % nrb;
         const uint32_t si = (j / nrb) * 8 + (b & 7);
-        if (si >= gw.hdr[0]) return;
+        S = &sets[si];
+        m = S->count;
         c_begin = 0;
         c_end = cols;
-        const WideSet& S = gw.sets[si];
-        first = S.first;
-        m = S.count;
         if constexpr (MODE == kWGateUp) {
-            pw[0] = S.p.gate;
-            ps[0] = S.p.gate_scale;
-            pw[kMats - 1] = S.p.up;
-            ps[kMats - 1] = S.p.up_scale;
+            pw[0] = S->p.gate;
+            ps[0] = S->p.gate_scale;
+            pw[kMats - 1] = S->p.up;
+            ps[kMats - 1] = S->p.up_scale;
         } else {
-            pw[0] = S.p.down;
-            ps[0] = S.p.down_scale;
+            pw[0] = S->p.down;
+            ps[0] = S->p.down_scale;
         }
+        if (si >= *set_count) return;  // the record (stale then) was requested along with the count
     }
     const uint32_t r0 = rb * kMatRows;
     const uint32_t nmt = (m + 15) / 16;  // vector tiles
-    // {act row, row of the split vectors} of member j (past m: the last)
+    // {act row, row of the split vectors} of member j
     auto member = [&](uint32_t j) -> uint2 {
-        const uint32_t i = first + (j < m ? j : m - 1);
-        if constexpr (MODE == kWGemv) return make_uint2(i, i);
-        const uint2 o = gw.order[i];
-        return MODE == kWGateUp ? o : make_uint2(o.x, o.x);
+        if constexpr (MODE == kWGemv) {
+            const uint32_t i = first + (j < m ? j : m - 1);
+            return make_uint2(i, i);
+        } else {
+            const uint32_t a = S->row[j];
+            if constexpr (MODE == kWDown) return make_uint2(a, a);
+            // the token of an act row: a / k by the reciprocal (a < 4096, k <= 32), or the
+            // shared expert's
+            return make_uint2(a, a < n_assign ? (a * g.k_inv) >> 20 : a - n_assign);
+        }
     };
     R mt[kMats];
     __amdgpu_buffer_rsrc_t rs[kMats];
@@ -271,7 +289,7 @@ __global__ __launch_bounds__(256, 3) void wide_products_kernel(
     const __amdgpu_buffer_rsrc_t rh = matrix_rsrc(vh), rl = matrix_rsrc(vl);
     const uint32_t wpitch = static_cast<uint32_t>(TR::wpitch(mt[0]));
     // this thread's units: weights (row, dword of the row segment), vectors (8 columns
-    // of kMT members)
+    // of kNA members)
     uint32_t woff[kNU], wlds[kNU];
     bool wlive[kNU];
 #pragma unroll
@@ -284,15 +302,18 @@ __global__ __launch_bounds__(256, 3) void wide_products_kernel(
         woff[i] = r * wpitch + 4 * d;
         wlds[i] = rr * L::kStride + d;
     }
-    const uint32_t ac = threadIdx.x & 15, am = threadIdx.x >> 4;
-    uint32_t aoff[kMT];
+    const uint32_t ac = threadIdx.x % kAUpr, am = threadIdx.x / kAUpr;
+    uint32_t aoff[kNA];
 #pragma unroll
-    for (uint32_t i = 0; i < kMT; ++i) aoff[i] = (member(am + 16 * i).y * cols + 8 * ac) * 2;
-    u32x4 sw[kMats][kNU], sa[2][kMT];
+    for (uint32_t i = 0; i < kNA; ++i) aoff[i] = (member(am + kAStep * i).y * cols + 8 * ac) * 2;
+    u32x4 sw[kMats][kNU], sa[kParts][kNA];
     uint32_t ssc[kMats] = {}, sts[kMats] = {};
+    // FP4 scales: dword c of row threadIdx.x / kSdw
+    constexpr uint32_t kSd = L::kSdw ? L::kSdw : 1;
+    const uint32_t s_row_l = threadIdx.x / kSd, s_c = threadIdx.x % kSd;
     auto stage = [&](uint32_t c0) {
-        const uint32_t kc = FULL || c_end - c0 >= kWChunk ? kWChunk : c_end - c0;
-        if (FULL || kc == kWChunk) {
+        const uint32_t kc = FULL || c_end - c0 >= kChunk ? kChunk : c_end - c0;
+        if (FULL || kc == kChunk) {
 #pragma unroll
             for (int t = 0; t < kMats; ++t) {
                 const int so = static_cast<int>(TR::wrow(mt[t], c0) - TR::wrow(mt[t], 0));
@@ -304,14 +325,16 @@ __global__ __launch_bounds__(256, 3) void wide_products_kernel(
                     }
             }
 #pragma unroll
-            for (uint32_t i = 0; i < kMT; ++i)
-                if (i < nmt) {
+            for (uint32_t i = 0; i < kNA; ++i)
+                if (kAStep * i / 16 < nmt) {
                     const auto q = __builtin_amdgcn_raw_buffer_load_b128(rh, static_cast<int>(aoff[i]), static_cast<int>(2 * c0), 0);
                     sa[0][i] = u32x4{q[0], q[1], q[2], q[3]};
-                    const auto p = __builtin_amdgcn_raw_buffer_load_b128(rl, static_cast<int>(aoff[i]), static_cast<int>(2 * c0), 0);
-                    sa[1][i] = u32x4{p[0], p[1], p[2], p[3]};
+                    if constexpr (kParts == 2) {
+                        const auto p = __builtin_amdgcn_raw_buffer_load_b128(rl, static_cast<int>(aoff[i]), static_cast<int>(2 * c0), 0);
+                        sa[1][i] = u32x4{p[0], p[1], p[2], p[3]};
+                    }
                 }
-        } else {  // a last chunk of 64 columns: half the units, shifted inside the row
+        } else {  // a short last chunk: the row's last unit shifted to end with it
             const uint32_t seg = TR::wdw(kc);
 #pragma unroll
             for (int t = 0; t < kMats; ++t) {
@@ -329,36 +352,38 @@ __global__ __launch_bounds__(256, 3) void wide_products_kernel(
                 }
             }
 #pragma unroll
-            for (uint32_t i = 0; i < kMT; ++i)
-                if (i < nmt && 8 * ac < kc) {
+            for (uint32_t i = 0; i < kNA; ++i)
+                if (kAStep * i / 16 < nmt && 8 * ac < kc) {
                     const auto q = __builtin_amdgcn_raw_buffer_load_b128(rh, static_cast<int>(aoff[i]), static_cast<int>(2 * c0), 0);
                     sa[0][i] = u32x4{q[0], q[1], q[2], q[3]};
-                    const auto p = __builtin_amdgcn_raw_buffer_load_b128(rl, static_cast<int>(aoff[i]), static_cast<int>(2 * c0), 0);
-                    sa[1][i] = u32x4{p[0], p[1], p[2], p[3]};
+                    if constexpr (kParts == 2) {
+                        const auto p = __builtin_amdgcn_raw_buffer_load_b128(rl, static_cast<int>(aoff[i]), static_cast<int>(2 * c0), 0);
+                        sa[1][i] = u32x4{p[0], p[1], p[2], p[3]};
+                    }
                 }
         }
-        if constexpr (TR::kScales) {  // one dword of E8M0 bytes per row
+        if constexpr (TR::kScales) {
 #pragma unroll
             for (int t = 0; t < kMats; ++t)
-                if (threadIdx.x < kMatRows) {
-                    const uint32_t r = r0 + threadIdx.x < rows ? r0 + threadIdx.x : rows - 1;
-                    ssc[t] = *as_global(reinterpret_cast<const uint32_t*>(TR::srow(mt[t], c0) +
-                                                                          static_cast<size_t>(r) * TR::spitch(mt[t])));
+                if (s_row_l < kMatRows && (FULL || s_c < TR::sdw(kc))) {
+                    const uint32_t r = r0 + s_row_l < rows ? r0 + s_row_l : rows - 1;
+                    ssc[t] = as_global(reinterpret_cast<const uint32_t*>(TR::srow(mt[t], c0) +
+                                                                         static_cast<size_t>(r) * TR::spitch(mt[t])))[s_c];
                 }
         }
         if constexpr (TR::kTileScale)
 #pragma unroll
-            for (int t = 0; t < kMats; ++t) sts[t] = TR::tile_scales(mt[t], r0, c0, kWChunk);
+            for (int t = 0; t < kMats; ++t) sts[t] = TR::tile_scales(mt[t], r0, c0, kc);
     };
     uint32_t ts_cur[kMats] = {};
     auto commit = [&](uint32_t c0) {
-        const uint32_t kc = FULL || c_end - c0 >= kWChunk ? kWChunk : c_end - c0;
+        const uint32_t kc = FULL || c_end - c0 >= kChunk ? kChunk : c_end - c0;
         typedef uint32_t u32x2s __attribute__((ext_vector_type(2), aligned(8)));
         typedef uint32_t u32x4s __attribute__((ext_vector_type(4), aligned(16)));
 #pragma unroll
         for (int t = 0; t < kMats; ++t) {
             uint32_t* base = wl + t * kMatRows * L::kStride;
-            if (FULL || kc == kWChunk) {
+            if (FULL || kc == kChunk) {
 #pragma unroll
                 for (uint32_t i = 0; i < kNU; ++i)
                     if ((kMatRows * kUpr) % 256 == 0 || wlive[i]) {
@@ -379,29 +404,30 @@ __global__ __launch_bounds__(256, 3) void wide_products_kernel(
                 }
             }
             if constexpr (TR::kScales)
-                if (threadIdx.x < kMatRows) sl[t * kMatRows + threadIdx.x] = ssc[t];
+                if (s_row_l < kMatRows) sl[t * kMatRows * kSd + threadIdx.x] = ssc[t];
             ts_cur[t] = sts[t];
         }
 #pragma unroll
-        for (uint32_t i = 0; i < kMT; ++i)
-            if (i < nmt && (FULL || 8 * ac < kc)) {
-                _Float16* dst = al + (am + 16 * i) * kWAStride + 8 * ac;
+        for (uint32_t i = 0; i < kNA; ++i)
+            if (kAStep * i / 16 < nmt && (FULL || 8 * ac < kc)) {
+                _Float16* dst = al + (am + kAStep * i) * L::kAStride + 8 * ac;
                 *reinterpret_cast<u32x4s*>(dst) = u32x4s{sa[0][i].x, sa[0][i].y, sa[0][i].z, sa[0][i].w};
-                *reinterpret_cast<u32x4s*>(dst + kWMembers * kWAStride) =
-                    u32x4s{sa[1][i].x, sa[1][i].y, sa[1][i].z, sa[1][i].w};
+                if constexpr (kParts == 2)
+                    *reinterpret_cast<u32x4s*>(dst + kMembers * L::kAStride) =
+                        u32x4s{sa[1][i].x, sa[1][i].y, sa[1][i].z, sa[1][i].w};
             }
     };
     // [row tile][vector tile]: the running sums of up to kFlush chunks, and of those
-    f32x4 acc[4][kMT], accl[4][kMT], total[4][kMT];
+    f32x4 acc[kRT][kMT], accl[kRT][kMT], total[kRT][kMT];
 #pragma unroll
-    for (int a = 0; a < 4; ++a)
+    for (int a = 0; a < kRT; ++a)
 #pragma unroll
         for (int b = 0; b < kMT; ++b) acc[a][b] = accl[a][b] = total[a][b] = f32x4{0.f, 0.f, 0.f, 0.f};
     // LDS row of this lane in row tile rt, and that tile's matrix
-    auto tile_mat = [&](int rt) { return MODE == kWGateUp ? rt >> 1 : 0; };
+    auto tile_mat = [&](int rt) { return MODE == kWGateUp ? rt / (kRT / 2) : 0; };
     auto tile_row = [&](int rt) {
-        return MODE == kWGateUp ? wr * 32u + static_cast<uint32_t>(rt & 1) * 16u + n16
-                                : wr * 64u + static_cast<uint32_t>(rt) * 16u + n16;
+        return MODE == kWGateUp ? wr * (8u * kRT) + static_cast<uint32_t>(rt % (kRT / 2)) * 16u + n16
+                                : wr * (16u * kRT) + static_cast<uint32_t>(rt) * 16u + n16;
     };
     // the products of block b of the chunk with vector tiles 0 .. MT - 1
     auto block = [&](uint32_t b, auto mtc) {
@@ -409,27 +435,30 @@ __global__ __launch_bounds__(256, 3) void wide_products_kernel(
         half8 xh[MT], xl[MT];
 #pragma unroll
         for (int v = 0; v < MT; ++v) {
-            const _Float16* src = al + (16u * v + n16) * kWAStride + 32u * b + 8u * kg;
+            const _Float16* src = al + (16u * v + n16) * L::kAStride + 32u * b + 8u * kg;
             xh[v] = *reinterpret_cast<const half8*>(src);
-            xl[v] = *reinterpret_cast<const half8*>(src + kWMembers * kWAStride);
+            if constexpr (kParts == 2) xl[v] = *reinterpret_cast<const half8*>(src + kMembers * L::kAStride);
         }
 #pragma unroll
-        for (int rt = 0; rt < 4; ++rt) {
+        for (int rt = 0; rt < kRT; ++rt) {
             const uint32_t lr = tile_mat(rt) * kMatRows + tile_row(rt);
             float sc;
             const half8 bw = TR::get(reinterpret_cast<const uint8_t*>(wl + lr * L::kStride),
-                                     reinterpret_cast<const uint8_t*>(sl + lr), ts_cur[tile_mat(rt)], b, kg, sc);
+                                     reinterpret_cast<const uint8_t*>(sl + lr * kSd), ts_cur[tile_mat(rt)], b, kg, sc);
             f32x4 zh[MT], zl[MT];
             const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
             for (int v = 0; v < MT; ++v) zh[v] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xh[v], bw, zero, 0, 0, 0);
+            if constexpr (kParts == 2)
 #pragma unroll
-            for (int v = 0; v < MT; ++v) zl[v] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xl[v], bw, zero, 0, 0, 0);
+                for (int v = 0; v < MT; ++v) zl[v] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xl[v], bw, zero, 0, 0, 0);
 #pragma unroll
             for (int v = 0; v < MT; ++v)
 #pragma unroll
                 for (int q = 0; q < 4; ++q) {
-                    if constexpr (kApart) {
+                    if constexpr (kParts == 1) {
+                        acc[rt][v][q] = __builtin_fmaf(sc, zh[v][q], acc[rt][v][q]);
+                    } else if constexpr (kApart) {
                         acc[rt][v][q] = __builtin_fmaf(sc, zh[v][q], acc[rt][v][q]);
                         accl[rt][v][q] = __builtin_fmaf(sc, zl[v][q], accl[rt][v][q]);
                     } else {
@@ -440,25 +469,25 @@ __global__ __launch_bounds__(256, 3) void wide_products_kernel(
     };
     uint32_t pending = 0;  // chunks in acc
     stage(c_begin);
-    for (uint32_t c0 = c_begin; c0 < c_end; c0 += kWChunk) {
-        const uint32_t kc = FULL || c_end - c0 >= kWChunk ? kWChunk : c_end - c0;
+    for (uint32_t c0 = c_begin; c0 < c_end; c0 += kChunk) {
+        const uint32_t kc = FULL || c_end - c0 >= kChunk ? kChunk : c_end - c0;
         __syncthreads();  // the previous chunk's (or set's) LDS reads are done
         commit(c0);
         __syncthreads();
-        if (c0 + kWChunk < c_end) stage(c0 + kWChunk);  // in flight during the products
+        if (c0 + kChunk < c_end) stage(c0 + kChunk);  // in flight during the products
         asm volatile("" ::: "memory");
         __builtin_amdgcn_sched_barrier(0);
-        const uint32_t per = FULL ? 2u : kc / 64;  // blocks of this wave's half
+        const uint32_t per = FULL ? kChunk / 64 : kc / 64;  // blocks of this wave's half
 #pragma unroll 1
         for (uint32_t i = 0; i < per; ++i) {
             const uint32_t b = wk * per + i;
             if (kMT == 1 || nmt > 1) block(b, std::integral_constant<int, kMT>{});
             else block(b, std::integral_constant<int, 1>{});
         }
-        if (++pending == (kApart ? 4 : kFlush)) {
+        if (++pending == kFlush) {
             pending = 0;
 #pragma unroll
-            for (int a = 0; a < 4; ++a)
+            for (int a = 0; a < kRT; ++a)
 #pragma unroll
                 for (int v = 0; v < kMT; ++v) {
                     if constexpr (kApart) acc[a][v] += accl[a][v];
@@ -467,13 +496,13 @@ __global__ __launch_bounds__(256, 3) void wide_products_kernel(
                 }
         }
     }
-    if (threadIdx.x < kWMembers) {
+    if (threadIdx.x < kMembers) {
         const uint2 o = member(threadIdx.x);
         s_row[threadIdx.x] = o.x;
-        s_mul[threadIdx.x] = vmult[o.y];
+        s_mul[threadIdx.x] = g.vmult[o.y];
     }
 #pragma unroll
-    for (int a = 0; a < 4; ++a)
+    for (int a = 0; a < kRT; ++a)
 #pragma unroll
         for (int v = 0; v < kMT; ++v) {
             if constexpr (kApart) acc[a][v] += accl[a][v];
@@ -481,13 +510,13 @@ __global__ __launch_bounds__(256, 3) void wide_products_kernel(
         }
     // the two column halves meet in LDS: wave (wr, wk) finishes vector tiles v with
     // v % 2 == wk and hands the others over
-    f32x4* const red = reinterpret_cast<f32x4*>(wl) + wr * 4 * kMT * 64;
+    f32x4* const red = reinterpret_cast<f32x4*>(wl) + wr * kRT * kMT * 64;
     __syncthreads();
 #pragma unroll
     for (int v = 0; v < kMT; ++v)
         if ((v & 1) != static_cast<int>(wk) && static_cast<uint32_t>(v) < nmt) {
 #pragma unroll
-            for (int rt = 0; rt < 4; ++rt) red[(v * 4 + rt) * 64 + lane] = total[rt][v];
+            for (int rt = 0; rt < kRT; ++rt) red[(v * kRT + rt) * 64 + lane] = total[rt][v];
         }
     __syncthreads();
     // lane: weight row n16 of the tile, members 16 v + 4 kg + q
@@ -495,7 +524,7 @@ __global__ __launch_bounds__(256, 3) void wide_products_kernel(
     for (int v = 0; v < kMT; ++v) {
         if ((v & 1) != static_cast<int>(wk) || static_cast<uint32_t>(v) >= nmt) continue;
 #pragma unroll
-        for (int rt = 0; rt < 4; ++rt) total[rt][v] += red[(v * 4 + rt) * 64 + lane];
+        for (int rt = 0; rt < kRT; ++rt) total[rt][v] += red[(v * kRT + rt) * 64 + lane];
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
             const uint32_t j = 16u * v + 4u * kg + static_cast<uint32_t>(q);
@@ -504,75 +533,211 @@ __global__ __launch_bounds__(256, 3) void wide_products_kernel(
                                              : static_cast<size_t>(s_row[j]) * rows;
             if constexpr (MODE == kWGateUp) {
 #pragma unroll
-                for (int h = 0; h < 2; ++h) {
+                for (int h = 0; h < kRT / 2; ++h) {
                     const uint32_t r = r0 + tile_row(h);
                     if (j < m && r < rows)
-                        out[at + r] = swiglu(total[h][v][q] * mul, total[h + 2][v][q] * mul, limit, official);
+                        g.out[at + r] = swiglu(total[h][v][q] * mul, total[h + kRT / 2][v][q] * mul, g.limit, g.official);
                 }
             } else {
 #pragma unroll
-                for (int rt = 0; rt < 4; ++rt) {
+                for (int rt = 0; rt < kRT; ++rt) {
                     const uint32_t r = r0 + tile_row(rt);
-                    if (j < m && r < rows) out[at + r] = total[rt][v][q] * mul;
+                    if (j < m && r < rows) g.out[at + r] = total[rt][v][q] * mul;
                 }
             }
         }
     }
 }
 
+template <class R, class K, int MODE, bool FULL>
+__global__ __launch_bounds__(256, K::kWaves) void wide_products_kernel(WideArgs g) {
+    wide_body<R, K, MODE, FULL>(g, g.n, g.sets, blockIdx.x);
+}
+
+// The official layer's products of a phase: the first n_sh workgroups take the FP8 shared
+// expert's sets (few, and the longest rows), the others the routed FP4 experts'. Apart
+// they took 37 + 254 us (gate/up) and 20 + 219 us (down) at 32 tokens of hidden 7168.
+template <class K, class KS, int MODE, bool FULL>
+__global__ __launch_bounds__(256, K::kWaves) void wide_pair_kernel(WideArgs g, const uint32_t* __restrict__ shared_n,
+                                                                   const WideSet* __restrict__ shared_sets,
+                                                                   uint32_t n_sh, uint32_t shared_nrb) {
+    if (blockIdx.x < n_sh) {
+        WideArgs h = g;
+        h.nrb = shared_nrb;
+        wide_body<Fp8Rows, KS, MODE, FULL>(h, shared_n, shared_sets, blockIdx.x);
+    } else {
+        wide_body<Fp4Rows, K, MODE, FULL>(g, g.n, g.sets, blockIdx.x - n_sh);
+    }
+}
+
 size_t al256(size_t v) { return (v + 255) & ~size_t(255); }
 
-template <class R, int MODE>
-void launch_wide_products(hipStream_t s, dim3 grid, WideWs gw, const void* w0, const void* s0, const _Float16* vh,
-                          const _Float16* vl, const float* vmult, float* dst, uint32_t cols, uint32_t rows,
-                          uint32_t n_vec, uint32_t range, uint32_t nrb, float limit, bool official) {
-    const size_t lds = 4 * static_cast<size_t>(WideLds<R>::kDwords);
-    if (Tile<R>::kScales || cols % kWChunk == 0)  // split FP4 rows are whole chunks
-        hipLaunchKernelGGL((wide_products_kernel<R, MODE, true>), grid, dim3(256), lds, s, gw, w0, s0, vh, vl, vmult, dst,
-                           cols, rows, n_vec, range, nrb, limit, official ? 1u : 0u);
-    else if constexpr (!Tile<R>::kScales)
-        hipLaunchKernelGGL((wide_products_kernel<R, MODE, false>), grid, dim3(256), lds, s, gw, w0, s0, vh, vl, vmult, dst,
-                           cols, rows, n_vec, range, nrb, limit, official ? 1u : 0u);
+template <class K, int MODE>
+uint32_t row_blocks(uint32_t rows) {
+    const uint32_t mr = MODE == kWGateUp ? K::kRows / 2 : K::kRows;
+    return (rows + mr - 1) / mr;
 }
 
-// One phase of the grouped experts: as many workgroups as there can be (row block,
-// set) pairs; a set's number is below max_sets, the real count is known on the device.
-template <class R, int MODE>
-void launch_wide_phase(hipStream_t s, WideWs gw, const _Float16* vh, const _Float16* vl, const float* vmult, float* dst,
-                       uint32_t cols, uint32_t rows, uint32_t max_sets, float limit,
-                       bool official) {
-    const uint32_t mr = MODE == kWGateUp ? kWRows / 2 : kWRows;
-    const uint32_t nrb = (rows + mr - 1) / mr;
-    launch_wide_products<R, MODE>(s, dim3(8 * nrb * ((max_sets + 7) / 8)), gw, nullptr, nullptr, vh, vl, vmult, dst, cols,
-                                  rows, 0, 0, nrb, limit, official);
+// Workgroups of a MoE phase: every (row block, set) pair there can be, in whole rounds of
+// the eight XCDs; a set's number is below max_sets, the real count is known on the device.
+uint32_t phase_blocks(uint32_t nrb, uint32_t max_sets) { return 8 * nrb * ((max_sets + 7) / 8); }
+
+template <class R, class K, int MODE>
+void launch_wide_products(hipStream_t s, dim3 grid, const WideArgs& g) {
+    const size_t lds = 4 * static_cast<size_t>(WideLds<R, K>::kDwords);
+    if (g.cols % K::kChunk == 0)
+        hipLaunchKernelGGL((wide_products_kernel<R, K, MODE, true>), grid, dim3(256), lds, s, g);
+    else
+        hipLaunchKernelGGL((wide_products_kernel<R, K, MODE, false>), grid, dim3(256), lds, s, g);
 }
 
-template <class R>
-void launch_wide_layer(hipStream_t s, WideWs gw, const _Float16* xh, const _Float16* xl, const float* xmult, float* act,
-                       _Float16* ah, _Float16* al, float* amult, float* part, uint32_t n_rows,
-                       uint32_t max_sets, uint32_t hidden, uint32_t inter, uint32_t out_dim, float limit) {
-    launch_wide_phase<R, kWGateUp>(s, gw, xh, xl, xmult, act, hidden, inter, max_sets, limit, false);
-    hipLaunchKernelGGL(wide_split_kernel, dim3(n_rows), dim3(256), 0, s, act, inter, ah, al, amult,
-                       Tile<R>::kPermuted ? 1u : 0u);
-    launch_wide_phase<R, kWDown>(s, gw, ah, al, amult, part, inter, out_dim, max_sets, 0.0f, false);
+template <class R, class K, int MODE>
+void launch_wide_phase(hipStream_t s, WideArgs g, uint32_t max_sets) {
+    g.nrb = row_blocks<K, MODE>(g.rows);
+    launch_wide_products<R, K, MODE>(s, dim3(phase_blocks(g.nrb, max_sets)), g);
+}
+
+template <class K, class KS, int MODE>
+void launch_wide_pair(hipStream_t s, WideArgs g, uint32_t max_sets, const uint32_t* shared_n,
+                      const WideSet* shared_sets, uint32_t max_shared) {
+    g.nrb = row_blocks<K, MODE>(g.rows);
+    const uint32_t nrb_s = row_blocks<KS, MODE>(g.rows), n_sh = phase_blocks(nrb_s, max_shared);
+    const uint32_t dw = WideLds<Fp4Rows, K>::kDwords > WideLds<Fp8Rows, KS>::kDwords ? WideLds<Fp4Rows, K>::kDwords
+                                                                                      : WideLds<Fp8Rows, KS>::kDwords;
+    const dim3 grid(n_sh + phase_blocks(g.nrb, max_sets));
+    static_assert(K::kChunk == KS::kChunk, "one FULL for both");
+    if (g.cols % K::kChunk == 0)
+        hipLaunchKernelGGL((wide_pair_kernel<K, KS, MODE, true>), grid, dim3(256), 4 * static_cast<size_t>(dw), s, g,
+                           shared_n, shared_sets, n_sh, nrb_s);
+    else
+        hipLaunchKernelGGL((wide_pair_kernel<K, KS, MODE, false>), grid, dim3(256), 4 * static_cast<size_t>(dw), s, g,
+                           shared_n, shared_sets, n_sh, nrb_s);
 }
 
 // Offsets in the kernels are 32-bit: matrices and split vectors below 2^31 bytes.
 bool below_2g(uint64_t rows, uint64_t bytes_per_row) { return rows * bytes_per_row < (uint64_t(1) << 31); }
 
+// Large work (128 weight rows per workgroup) where the matrices are large and an expert
+// has many vectors; 64 rows otherwise (more workgroups, a shorter chain of chunks each).
+// us per layer, large / small: Q4_0 2048 x 768, 128 experts, top-8 at 512 tokens 366 /
+// 376, at 200 181 / 178; Q4_0 4096 x 1536, 64 experts at 256 tokens 505 / 543, at 40 280 /
+// 233; IQ3_0 2048 x 2048 at 300 tokens 443 / 520; Q4_0 1024 x 512, 16 experts at 250 tokens
+// 63 / 59. Split FP4 work items hold 16 vectors in both: from about one vector per expert
+// of very large matrices (7168 x 2048, 64 experts, 32 tokens 411 / 435; official, 256
+// experts, 6 tokens 195 / 187).
+bool large_work(bool fp4, uint64_t rows, uint64_t cols, uint64_t n_assign, uint64_t n_table) {
+    return (n_assign >= 16 * n_table && rows * cols >= (uint64_t(1) << 20)) ||
+           (fp4 && n_assign >= n_table && rows * cols >= (uint64_t(8) << 20));
+}
+
+uint32_t most_sets(uint32_t a, uint32_t n_table, uint32_t members) { return (a < n_table ? a : n_table) + a / members; }
+
+// The workspace of one launch of the layer.
+struct LayerWs {
+    uint32_t* hdr;
+    WideSet *sets, *shared_sets;
+    float *xd, *xmult, *amult, *act, *part;
+    _Float16 *xh, *xl, *ah, *al;
+};
+int32_t layer_workspace(objeta_hip_context* ctx, hipStream_t s, uint64_t T, uint64_t NR, uint32_t n_sets,
+                        uint32_t n_shared, uint64_t H, uint64_t I, uint64_t O, bool official, LayerWs& w) {
+    size_t off = 0;
+    auto take = [&](size_t bytes) {
+        const size_t at = off;
+        off += al256(bytes);
+        return at;
+    };
+    const size_t o_hdr = take(16);
+    const size_t o_set = take(sizeof(WideSet) * ((n_sets + 7) & ~7u));
+    const size_t o_ssh = take(sizeof(WideSet) * ((n_shared + 7) & ~7u));
+    const size_t o_xd = take(official ? 4 * T * H : 0);
+    const size_t o_xm = take(4 * T), o_am = take(4 * NR);
+    const size_t o_xh = take(2 * T * H), o_xl = take(official ? 0 : 2 * T * H);
+    const size_t o_act = take(4 * NR * I), o_ah = take(2 * NR * I), o_al = take(official ? 0 : 2 * NR * I);
+    const size_t o_part = take(4 * NR * O);
+    void* p = nullptr;
+    OBJ_TRY(ensure_workspace(ctx, s, kWsGrouped, off, &p));
+    char* b = static_cast<char*>(p);
+    w.hdr = reinterpret_cast<uint32_t*>(b + o_hdr);
+    w.sets = reinterpret_cast<WideSet*>(b + o_set);
+    w.shared_sets = reinterpret_cast<WideSet*>(b + o_ssh);
+    w.xd = reinterpret_cast<float*>(b + o_xd);
+    w.xmult = reinterpret_cast<float*>(b + o_xm);
+    w.amult = reinterpret_cast<float*>(b + o_am);
+    w.xh = reinterpret_cast<_Float16*>(b + o_xh);
+    w.xl = official ? nullptr : reinterpret_cast<_Float16*>(b + o_xl);
+    w.act = reinterpret_cast<float*>(b + o_act);
+    w.ah = reinterpret_cast<_Float16*>(b + o_ah);
+    w.al = official ? nullptr : reinterpret_cast<_Float16*>(b + o_al);
+    w.part = reinterpret_cast<float*>(b + o_part);
+    return 0;
+}
+
+uint32_t reciprocal(uint64_t k) { return static_cast<uint32_t>(((uint64_t(1) << 20) + k - 1) / k); }
+
+WideArgs gate_up_args(const LayerWs& w, uint32_t hidden, uint32_t inter, uint64_t k, uint32_t a, float limit, bool official) {
+    WideArgs g{};
+    g.n = w.hdr;
+    g.sets = w.sets;
+    g.vh = w.xh;
+    g.vl = w.xl;
+    g.vmult = w.xmult;
+    g.out = w.act;
+    g.cols = hidden;
+    g.rows = inter;
+    g.k_inv = reciprocal(k);
+    g.n_assign = a;
+    g.limit = limit;
+    g.official = official ? 1u : 0u;
+    return g;
+}
+
+WideArgs down_args(const LayerWs& w, uint32_t inter, uint32_t out_dim, uint32_t a) {
+    WideArgs g{};
+    g.n = w.hdr;
+    g.sets = w.sets;
+    g.vh = w.ah;
+    g.vl = w.al;
+    g.vmult = w.amult;
+    g.out = w.part;
+    g.cols = inter;
+    g.rows = out_dim;
+    g.n_assign = a;
+    return g;
+}
+
+bool wide_shape(int32_t format, uint64_t n_table, uint64_t k, uint64_t hidden, uint64_t inter, uint64_t out_dim) {
+    if (format < OBJETA_HIP_Q4_0 || format > OBJETA_HIP_FP4_E2M1) return false;
+    if (k == 0 || k > 32 || n_table == 0 || n_table > kWMaxTable || out_dim == 0) return false;
+    if (hidden == 0 || inter == 0 || hidden % 64 || inter % 64 || hidden > (1u << 20) || inter > (1u << 20) ||
+        out_dim > (1u << 20))
+        return false;
+    return format != OBJETA_HIP_FP4_E2M1 || (hidden % 128 == 0 && inter % 128 == 0);
+}
+
+// Matrices of at most 2^31 bytes (FP8, the widest of the formats, when `official`).
+bool matrices_fit(int32_t format, bool official, uint64_t hidden, uint64_t inter, uint64_t out_dim) {
+    const uint64_t per32 = official ? 32 : format == OBJETA_HIP_Q4_0 ? 18 : format == OBJETA_HIP_Q5_0 ? 22
+                         : format == OBJETA_HIP_IQ3_0 ? 14 : 16;
+    return below_2g(inter, hidden / 32 * per32) && below_2g(out_dim, inter / 32 * per32);
+}
+
+// Tokens of one launch: at most kWMaxAssign assignments, split vectors below 2^31 bytes.
+uint64_t launch_tokens(uint64_t k, uint64_t hidden, uint64_t inter) {
+    const uint64_t lim = (uint64_t(1) << 31) - 1;
+    uint64_t t = kWMaxAssign / k;
+    if (t > lim / (2 * hidden)) t = lim / (2 * hidden);
+    if (t > lim / (2 * inter * (k + 1))) t = lim / (2 * inter * (k + 1));
+    return t;
+}
+
 }  // namespace
 
 bool wide_supported(int32_t format, uint64_t n_table, uint64_t n_tokens, uint64_t k, uint64_t hidden, uint64_t inter,
                     uint64_t out_dim) {
-    if (format < OBJETA_HIP_Q4_0 || format > OBJETA_HIP_FP4_E2M1) return false;
-    if (k == 0 || k > 32 || n_table == 0 || n_table > kWMaxTable || n_tokens < kWideMinTokens || out_dim == 0) return false;
-    if (hidden == 0 || inter == 0 || hidden % 64 || inter % 64 || hidden > (1u << 20) || inter > (1u << 20) ||
-        out_dim > (1u << 20))
-        return false;
-    if (format == OBJETA_HIP_FP4_E2M1 && (hidden % 128 || inter % 128)) return false;
-    const uint64_t t = n_tokens < kWMaxAssign / k ? n_tokens : kWMaxAssign / k;  // tokens of a launch
-    return below_2g(inter, hidden) && below_2g(out_dim, inter) && below_2g(t, 2 * hidden) &&
-           below_2g(t * (k + 1), 2 * inter);
+    if (n_tokens < (format == OBJETA_HIP_FP4_E2M1 ? 1 : kWideMinTokens)) return false;
+    return wide_shape(format, n_table, k, hidden, inter, out_dim) && matrices_fit(format, false, hidden, inter, out_dim) &&
+           launch_tokens(k, hidden, inter) > 0;
 }
 
 int32_t launch_moe_wide(objeta_hip_context* ctx, int32_t format, hipStream_t s, const objeta_hip_expert_ptrs* table,
@@ -585,61 +750,123 @@ int32_t launch_moe_wide(objeta_hip_context* ctx, int32_t format, hipStream_t s, 
     if (!table || !ids || !wts || !x || !out) OBJ_FAIL(kInvalidInput, action, "NULL device pointer");
     if (reinterpret_cast<uintptr_t>(x) % 16) OBJ_FAIL(kInvalidInput, action, "x must be 16-byte aligned");
     const uint32_t H = static_cast<uint32_t>(hidden), I = static_cast<uint32_t>(inter), O = static_cast<uint32_t>(out_dim);
-    const uint32_t M = format == OBJETA_HIP_FP4_E2M1 ? kWMembersOf<Fp4Rows> : kWMembersOf<QRows<kQ4>>;
     const uint32_t kk = static_cast<uint32_t>(k), E = static_cast<uint32_t>(n_table);
-    // tokens in equal slices of at most kWMaxAssign assignments (the workspace of a
-    // slice is reused by the next)
-    const uint64_t per = kWMaxAssign / k, slices = (n_tokens + per - 1) / per;
+    const bool fp4 = format == OBJETA_HIP_FP4_E2M1, large = large_work(fp4, inter, hidden, n_tokens * k, n_table);
+    const uint32_t M = large && !fp4 ? WorkLarge::kMembers : WorkSmall::kMembers;
+    // tokens in equal slices (the workspace of a slice is reused by the next)
+    const uint64_t per = launch_tokens(k, hidden, inter), slices = (n_tokens + per - 1) / per;
     const uint64_t slice = (n_tokens + slices - 1) / slices;
-    const uint32_t T = static_cast<uint32_t>(slice), A = T * kk;
-    const uint32_t NR = A + (shared ? T : 0);  // act rows: routed, then shared
-    const uint32_t NS = (A < E ? A : E) + A / M + (shared ? (T + M - 1) / M : 0);
-    size_t off = 0;
-    const size_t o_hdr = off; off += al256(16);
-    const size_t o_set = off; off += al256(sizeof(WideSet) * NS);
-    const size_t o_ord = off; off += al256(8ull * NR);
-    const size_t o_xm = off; off += al256(4ull * T);
-    const size_t o_am = off; off += al256(4ull * NR);
-    const size_t o_xh = off; off += al256(2ull * T * H);
-    const size_t o_xl = off; off += al256(2ull * T * H);
-    const size_t o_act = off; off += al256(4ull * NR * I);
-    const size_t o_ah = off; off += al256(2ull * NR * I);
-    const size_t o_all = off; off += al256(2ull * NR * I);
-    const size_t o_part = off; off += al256(4ull * NR * O);
-    void* wsp = nullptr;
-    OBJ_TRY(ensure_workspace(ctx, s, kWsGrouped, off, &wsp));
-    char* b = static_cast<char*>(wsp);
-    const WideWs gw{reinterpret_cast<uint32_t*>(b + o_hdr), reinterpret_cast<WideSet*>(b + o_set),
-                    reinterpret_cast<uint2*>(b + o_ord)};
-    float* xmult = reinterpret_cast<float*>(b + o_xm);
-    float* amult = reinterpret_cast<float*>(b + o_am);
-    auto* xh = reinterpret_cast<_Float16*>(b + o_xh);
-    auto* xl = reinterpret_cast<_Float16*>(b + o_xl);
-    float* act = reinterpret_cast<float*>(b + o_act);
-    auto* ah = reinterpret_cast<_Float16*>(b + o_ah);
-    auto* all = reinterpret_cast<_Float16*>(b + o_all);
-    float* part = reinterpret_cast<float*>(b + o_part);
-    const bool perm = format == OBJETA_HIP_FP4_E2M1 ? Tile<Fp4Rows>::kPermuted : Tile<QRows<kQ4>>::kPermuted;
+    auto sets_of = [&](uint64_t t) {
+        return most_sets(static_cast<uint32_t>(t) * kk, E, M) + (shared ? static_cast<uint32_t>((t + M - 1) / M) : 0u);
+    };
+    LayerWs w;
+    OBJ_TRY(layer_workspace(ctx, s, slice, slice * k + (shared ? slice : 0), sets_of(slice), 0, hidden, inter, out_dim,
+                            false, w));
+    const bool perm = fp4 ? Tile<Fp4Rows>::kPermuted : Tile<QRows<kQ4>>::kPermuted;
     for (uint64_t t0 = 0; t0 < n_tokens; t0 += slice) {
         const uint32_t t = static_cast<uint32_t>(n_tokens - t0 < slice ? n_tokens - t0 : slice), a = t * kk;
-        const uint32_t nr = a + (shared ? t : 0);
-        const uint32_t ns = (a < E ? a : E) + a / M + (shared ? (t + M - 1) / M : 0);
+        const uint32_t ns = sets_of(t);
         const uint32_t* idt = ids + t0 * k;
-        hipLaunchKernelGGL(wide_prepare_kernel, dim3(1 + t), dim3(256), 0, s, idt, a, E, table, shared, t, kk, M, gw,
-                           ctx->err_word, x + t0 * hidden, H, xh, xl, xmult, perm ? 1u : 0u);
-#define OBJ_WIDE(R) \
-    launch_wide_layer<R>(s, gw, xh, xl, xmult, act, ah, all, amult, part, nr, ns, H, I, O, limit)
+        hipLaunchKernelGGL(wide_prepare_kernel, dim3(1 + t), dim3(256), 0, s, idt, a, E, table, shared, t, M, w.hdr, w.sets,
+                           static_cast<WideSet*>(nullptr), ctx->err_word, x + t0 * hidden, H, w.xh, w.xl, w.xmult,
+                           perm ? 1u : 0u);
+        const WideArgs gu = gate_up_args(w, H, I, k, a, limit, false), dn = down_args(w, I, O, a);
+        const uint32_t nr = a + (shared ? t : 0);
+#define OBJ_WIDE_LAYER(R, K)                                                                                         {                                                                                                                    launch_wide_phase<R, K, kWGateUp>(s, gu, ns);                                                                    hipLaunchKernelGGL(wide_split_kernel, dim3(nr), dim3(256), 0, s, w.act, I, w.ah, w.al, w.amult,                                    perm ? 1u : 0u);                                                                              launch_wide_phase<R, K, kWDown>(s, dn, ns);                                                                  }
         switch (format) {
-            case OBJETA_HIP_Q4_0: OBJ_WIDE(QRows<kQ4>); break;
-            case OBJETA_HIP_Q5_0: OBJ_WIDE(QRows<kQ5>); break;
-            case OBJETA_HIP_IQ3_0: OBJ_WIDE(QRows<kIQ3>); break;
-            default: OBJ_WIDE(Fp4Rows); break;
+            case OBJETA_HIP_Q4_0:
+                if (large) OBJ_WIDE_LAYER(QRows<kQ4>, WorkLarge) else OBJ_WIDE_LAYER(QRows<kQ4>, WorkSmall)
+                break;
+            case OBJETA_HIP_Q5_0:
+                if (large) OBJ_WIDE_LAYER(QRows<kQ5>, WorkLarge) else OBJ_WIDE_LAYER(QRows<kQ5>, WorkSmall)
+                break;
+            case OBJETA_HIP_IQ3_0:
+                if (large) OBJ_WIDE_LAYER(QRows<kIQ3>, WorkLarge) else OBJ_WIDE_LAYER(QRows<kIQ3>, WorkSmall)
+                break;
+            default:
+                if (large) OBJ_WIDE_LAYER(Fp4Rows, WorkLarge4) else OBJ_WIDE_LAYER(Fp4Rows, WorkSmall)
+                break;
         }
-#undef OBJ_WIDE
-        launch_moe_combine(s, idt, wts + t0 * k, part, shared ? part + static_cast<size_t>(a) * O : nullptr,
+#undef OBJ_WIDE_LAYER
+        launch_moe_combine(s, idt, wts + t0 * k, w.part, shared ? w.part + static_cast<size_t>(a) * O : nullptr,
                            resid ? resid + t0 * out_dim : nullptr, out + t0 * out_dim, t, kk, O, E);
         OBJ_HIP(hipGetLastError(), action);
     }
+    return 0;
+}
+
+bool official_grouped_supported(uint64_t n_table, uint64_t n_tokens, uint64_t k, uint64_t hidden, uint64_t inter,
+                                uint64_t out_dim) {
+    return n_tokens >= kOfficialGroupedMinTokens && wide_shape(OBJETA_HIP_FP4_E2M1, n_table, k, hidden, inter, out_dim) &&
+           matrices_fit(OBJETA_HIP_FP4_E2M1, true, hidden, inter, out_dim) && n_tokens <= launch_tokens(k, hidden, inter);
+}
+
+// The official layer of launch_moe_official_fp4 on the grouped products: x is quantized
+// and dequantized as there (its values, a 4-bit significand times a power of two, are
+// their own fp16 high part: what lies below 2^-38 of the row's largest value, past the
+// fp16 subnormals, is dropped, far below the last bit of the fp32 sums), the routed FP4
+// experts and the FP8 shared expert read each matrix once per member set, in one launch
+// per phase unless the caller times them apart (marks), the intermediates are quantized
+// in place, and the combine adds w * down in slot order from zero, then the shared
+// expert's down.
+int32_t launch_moe_official_grouped(objeta_hip_context* ctx, hipStream_t s, const objeta_hip_expert_ptrs* table,
+                                    uint64_t n_table, const objeta_hip_expert_ptrs* shared, const uint32_t* ids,
+                                    const float* wts, uint64_t n_tokens, uint64_t k, const float* x, float* out,
+                                    uint64_t hidden, uint64_t inter, uint64_t out_dim, float limit,
+                                    uint8_t* inter_values, uint8_t* inter_scales, const OfficialMarks* marks) {
+    const char* action = "launch official FP4 MoE (grouped)";
+    // the routed FP4 and the shared FP8 sets multiply the same split activations
+    static_assert(Tile<Fp4Rows>::kPermuted == Tile<Fp8Rows>::kPermuted, "one activation order for both tiles");
+    if (!official_grouped_supported(n_table, n_tokens, k, hidden, inter, out_dim))
+        OBJ_FAIL(kUnsupported, action, "shape outside the grouped official path");
+    const uint32_t T = static_cast<uint32_t>(n_tokens), A = static_cast<uint32_t>(n_tokens * k);
+    const uint32_t NR = A + (shared ? T : 0);  // act rows: routed, then shared
+    const uint32_t M = WorkOfficial::kMembers;
+    const uint32_t NS = most_sets(A, static_cast<uint32_t>(n_table), M), NSS = shared ? (T + M - 1) / M : 0;
+    const uint32_t H = static_cast<uint32_t>(hidden), I = static_cast<uint32_t>(inter), O = static_cast<uint32_t>(out_dim);
+    LayerWs w;
+    OBJ_TRY(layer_workspace(ctx, s, T, NR, NS, NSS, hidden, inter, out_dim, true, w));
+    auto mark = [&](hipEvent_t e) -> int32_t {
+        if (e) OBJ_HIP(hipEventRecord(e, s), "record event");
+        return 0;
+    };
+    const bool large = large_work(true, inter, hidden, A, n_table), apart = marks != nullptr;
+    const uint32_t perm = Tile<Fp4Rows>::kPermuted ? 1u : 0u;
+    OBJ_TRY(launch_act_quant(s, x, T, H, nullptr, nullptr, w.xd));
+    hipLaunchKernelGGL(wide_prepare_kernel, dim3(1 + T), dim3(256), 0, s, ids, A, static_cast<uint32_t>(n_table), table,
+                       shared, T, M, w.hdr, w.sets, w.shared_sets, ctx->err_word, w.xd, H, w.xh, w.xl, w.xmult, perm);
+    const WideArgs gu = gate_up_args(w, H, I, k, A, limit, true), dn = down_args(w, I, O, A);
+    auto shared_args = [&](WideArgs g) {
+        g.n = w.hdr + 1;
+        g.sets = w.shared_sets;
+        return g;
+    };
+    if (shared && !apart) {
+        if (large) launch_wide_pair<WorkOfficial, WorkOfficialSmall, kWGateUp>(s, gu, NS, w.hdr + 1, w.shared_sets, NSS);
+        else launch_wide_pair<WorkOfficialSmall, WorkOfficialSmall, kWGateUp>(s, gu, NS, w.hdr + 1, w.shared_sets, NSS);
+    } else {
+        if (large) launch_wide_phase<Fp4Rows, WorkOfficial, kWGateUp>(s, gu, NS);
+        else launch_wide_phase<Fp4Rows, WorkOfficialSmall, kWGateUp>(s, gu, NS);
+        OBJ_TRY(mark(marks ? marks->gate_up_end : nullptr));
+        if (shared) launch_wide_phase<Fp8Rows, WorkOfficialSmall, kWGateUp>(s, shared_args(gu), NSS);
+        OBJ_TRY(mark(marks ? marks->shared_gate_up_end : nullptr));
+    }
+    OBJ_HIP(hipGetLastError(), action);
+    OBJ_TRY(launch_act_quant(s, w.act, NR, I, inter_values, inter_scales, w.act));
+    OBJ_TRY(mark(marks ? marks->act_quant_end : nullptr));
+    hipLaunchKernelGGL(wide_split_kernel, dim3(NR), dim3(256), 0, s, w.act, I, w.ah, w.al, w.amult, perm);
+    if (shared && !apart) {
+        if (large) launch_wide_pair<WorkOfficial, WorkOfficialSmall, kWDown>(s, dn, NS, w.hdr + 1, w.shared_sets, NSS);
+        else launch_wide_pair<WorkOfficialSmall, WorkOfficialSmall, kWDown>(s, dn, NS, w.hdr + 1, w.shared_sets, NSS);
+    } else {
+        if (large) launch_wide_phase<Fp4Rows, WorkOfficial, kWDown>(s, dn, NS);
+        else launch_wide_phase<Fp4Rows, WorkOfficialSmall, kWDown>(s, dn, NS);
+        OBJ_TRY(mark(marks ? marks->down_end : nullptr));
+        if (shared) launch_wide_phase<Fp8Rows, WorkOfficialSmall, kWDown>(s, shared_args(dn), NSS);
+    }
+    launch_moe_combine(s, ids, wts, w.part, shared ? w.part + static_cast<size_t>(A) * O : nullptr, nullptr, out, T,
+                       static_cast<uint32_t>(k), O, static_cast<uint32_t>(n_table));
+    OBJ_HIP(hipGetLastError(), action);
     return 0;
 }
 
@@ -647,47 +874,68 @@ bool gemv_wide_supported(int32_t format, uint64_t rows, uint64_t cols, uint64_t 
     return batch >= kGemvWideMinBatch && below_2g(rows, cols) && below_2g(batch, 2 * cols) && (batch + 15) / 16 <= 65535;
 }
 
-int32_t launch_gemv_wide(objeta_hip_context* ctx, hipStream_t s, int32_t format, const void* w, const void* ws,
-                         const float* x, float* y, uint64_t rows, uint64_t cols, uint64_t batch) {
-    const char* action = "launch batched GEMV (wide)";
-    const uint32_t R = static_cast<uint32_t>(rows), K = static_cast<uint32_t>(cols), B = static_cast<uint32_t>(batch);
+namespace {
+
+template <class R, class K>
+int32_t launch_gemv_wide_t(objeta_hip_context* ctx, hipStream_t s, const void* w, const void* ws, const float* x, float* y,
+                           uint32_t rows, uint32_t cols, uint32_t batch) {
     const uint32_t cus = ctx->info.compute_units > 0 ? static_cast<uint32_t>(ctx->info.compute_units) : 256u;
-    const uint32_t M = format == OBJETA_HIP_FP4_E2M1 ? kWMembersOf<Fp4Rows> : kWMembersOf<QRows<kQ4>>;
-    const uint32_t nrb = (R + kWRows - 1) / kWRows, ng = (B + M - 1) / M;
-    // column ranges for about two workgroups per CU, of at least four chunks
-    const uint32_t chunks = (K + kWChunk - 1) / kWChunk;
+    const uint32_t nrb = row_blocks<K, kWGemv>(rows), ng = (batch + K::kMembers - 1) / K::kMembers;
+    // column ranges for about two workgroups per CU, of at least 512 columns (in units of
+    // the larger chunk)
+    const uint32_t units = (cols + 255) / 256;
     uint32_t ks = (2 * cus + nrb * ng - 1) / (nrb * ng);
-    if (ks > (chunks + 3) / 4) ks = (chunks + 3) / 4;
-    const uint32_t rc = (chunks + ks - 1) / ks;  // chunks per range
-    ks = (chunks + rc - 1) / rc;
+    if (ks > (units + 1) / 2) ks = (units + 1) / 2;
+    WideArgs g{};
+    g.range = 256 * ((units + ks - 1) / ks);
+    ks = (cols + g.range - 1) / g.range;
     size_t off = 0;
-    const size_t o_xm = off; off += al256(4ull * B);
-    const size_t o_xh = off; off += al256(2ull * B * K);
-    const size_t o_xl = off; off += al256(2ull * B * K);
-    const size_t o_part = off; off += ks > 1 ? al256(4ull * ks * B * R) : 0;
+    const size_t o_xm = off; off += al256(4ull * batch);
+    const size_t o_xh = off; off += al256(2ull * batch * cols);
+    const size_t o_xl = off; off += al256(2ull * batch * cols);
+    const size_t o_part = off; off += ks > 1 ? al256(4ull * ks * batch * rows) : 0;
     void* wsp = nullptr;
     OBJ_TRY(ensure_workspace(ctx, s, kWsGemv, off, &wsp));
     char* b = static_cast<char*>(wsp);
     float* xmult = reinterpret_cast<float*>(b + o_xm);
     auto* xh = reinterpret_cast<_Float16*>(b + o_xh);
     auto* xl = reinterpret_cast<_Float16*>(b + o_xl);
-    float* part = ks > 1 ? reinterpret_cast<float*>(b + o_part) : y;
-    const bool perm = format == OBJETA_HIP_FP4_E2M1 ? Tile<Fp4Rows>::kPermuted : Tile<QRows<kQ4>>::kPermuted;
-    hipLaunchKernelGGL(wide_split_kernel, dim3(B), dim3(256), 0, s, x, K, xh, xl, xmult, perm ? 1u : 0u);
-    const dim3 grid(nrb, ks, ng);
-#define OBJ_WIDE(RT)                                                                                                  \
-    launch_wide_products<RT, kWGemv>(s, grid, WideWs{}, w, ws, xh, xl, xmult, part, K, R, B, rc * kWChunk, nrb, 0.0f, \
-                                     false)
+    g.w0 = w;
+    g.s0 = ws;
+    g.vh = xh;
+    g.vl = xl;
+    g.vmult = xmult;
+    g.out = ks > 1 ? reinterpret_cast<float*>(b + o_part) : y;
+    g.cols = cols;
+    g.rows = rows;
+    g.n_vec = batch;
+    g.nrb = nrb;
+    hipLaunchKernelGGL(wide_split_kernel, dim3(batch), dim3(256), 0, s, x, cols, xh, xl, xmult,
+                       Tile<R>::kPermuted ? 1u : 0u);
+    launch_wide_products<R, K, kWGemv>(s, dim3(nrb, ks, ng), g);
+    if (ks > 1) launch_gemv_reduce(s, g.out, y, rows, batch, ks);
+    OBJ_HIP(hipGetLastError(), "launch batched GEMV (wide)");
+    return 0;
+}
+
+}  // namespace
+
+int32_t launch_gemv_wide(objeta_hip_context* ctx, hipStream_t s, int32_t format, const void* w, const void* ws,
+                         const float* x, float* y, uint64_t rows, uint64_t cols, uint64_t batch) {
+    const uint32_t R = static_cast<uint32_t>(rows), C = static_cast<uint32_t>(cols), B = static_cast<uint32_t>(batch);
+    // us, large / small work: Q5_0 14336 x 4096 by 32 vectors 37.5 / 41.8, Q4_0 4096 x 4096
+    // by 64 25.5 / 24.5, split FP4 5000 x 3584 by 100 36.3 / 34.4
+    const bool large = B > WorkSmall::kMembers && rows * cols >= (uint64_t(1) << 25);
+#define OBJ_WIDE(RT, KL)                                                                       \
+    (large ? launch_gemv_wide_t<RT, KL>(ctx, s, w, ws, x, y, R, C, B)                          \
+           : launch_gemv_wide_t<RT, WorkSmall>(ctx, s, w, ws, x, y, R, C, B))
     switch (format) {
-        case OBJETA_HIP_Q4_0: OBJ_WIDE(QRows<kQ4>); break;
-        case OBJETA_HIP_Q5_0: OBJ_WIDE(QRows<kQ5>); break;
-        case OBJETA_HIP_IQ3_0: OBJ_WIDE(QRows<kIQ3>); break;
-        default: OBJ_WIDE(Fp4Rows); break;
+        case OBJETA_HIP_Q4_0: return OBJ_WIDE(QRows<kQ4>, WorkLarge);
+        case OBJETA_HIP_Q5_0: return OBJ_WIDE(QRows<kQ5>, WorkLarge);
+        case OBJETA_HIP_IQ3_0: return OBJ_WIDE(QRows<kIQ3>, WorkLarge);
+        default: return OBJ_WIDE(Fp4Rows, WorkLarge4);
     }
 #undef OBJ_WIDE
-    if (ks > 1) launch_gemv_reduce(s, part, y, R, B, ks);
-    OBJ_HIP(hipGetLastError(), action);
-    return 0;
 }
 
 }  // namespace objeta

@@ -1,7 +1,8 @@
 """Products with many vectors (wide.hip) on the GPU: the batched GEMV from 9 vectors and
-the experts of a layer from 32 tokens, against the CPU oracle. Work items hold 32 vectors
-(16 for split FP4), workgroups 128 weight rows (64 of gate and of up) and 128-column
-chunks, launches 4096 assignments; the sizes lie at the edges of these."""
+the experts of a layer from 9 tokens, against the CPU oracle. Work items hold 16 vectors and
+workgroups 64 weight rows (32 of gate and of up) in 256-column chunks; for large matrices
+with many vectors 32 (split FP4: 16), 128 and 128 (256); launches take 4096 assignments. The
+sizes lie at the edges of these."""
 import ctypes as C
 
 import numpy as np
@@ -34,6 +35,22 @@ def test_gemv_wide(backend, fmt, rows, cols, batch):
                                         QGemvShape.new(fmt, rows, cols), batch=batch)
     y = dy.download(np.float32, batch * rows).reshape(batch, rows)
     for t in range(batch):
+        xt = xs[t * cols:(t + 1) * cols]
+        _assert_close(y[t], orc.gemv(int(fmt), q, xt, rows, cols), q, xt, fmt, rows, cols)
+
+
+@pytest.mark.parametrize("fmt,cols", [(QuantFormat.Q4_0, 4096), (QuantFormat.Q5_0, 4160), (QuantFormat.IQ3_0, 4096)])
+def test_gemv_wide_large_matrix(backend, fmt, cols):
+    """8260 rows: the large work, the last row block 68 rows deep, a second work item of one
+    vector, and (4160 columns) a short last chunk."""
+    rows, batch = 8260, 33
+    q = orc.quantize_matrix(int(fmt), orc.gauss(rows * cols, 90, 0.02), rows, cols)
+    xs = orc.gauss(batch * cols, 91, 1.0)
+    dy = backend.alloc(batch * rows * 4)
+    QuantBackend(backend).launch_kernel(fmt, None, backend.to_device(q), backend.to_device(xs), dy,
+                                        QGemvShape.new(fmt, rows, cols), batch=batch)
+    y = dy.download(np.float32, batch * rows).reshape(batch, rows)
+    for t in (0, 15, 16, 31, 32):
         xt = xs[t * cols:(t + 1) * cols]
         _assert_close(y[t], orc.gemv(int(fmt), q, xt, rows, cols), q, xt, fmt, rows, cols)
 
@@ -79,14 +96,18 @@ def test_gemv_wide_non_finite_and_extreme_vectors(backend):
 
 
 @pytest.mark.parametrize("fmt,E,K,T,H,I,shared", [
-    (Q4, 16, 4, 32, 256, 128, False),     # the smallest batch
+    (Q4, 16, 4, 9, 256, 128, False),      # the smallest batch
     (Q5, 3, 2, 33, 192, 64, True),        # short chunks, inter of one row block
     (IQ3, 7, 3, 70, 320, 192, True),
     (FP4, 5, 4, 65, 256, 384, True),
     (Q4, 6, 4, 1030, 64, 64, True),       # two launches' worth of assignments
+    (Q4, 2, 2, 33, 1024, 1024, False),    # the large work: two vector tiles, and one over
+    (Q5, 2, 1, 47, 1088, 1024, True),     # with a short chunk
+    (IQ3, 2, 2, 70, 1024, 1088, False),   # with ragged row blocks
+    (FP4, 2, 2, 40, 1152, 1024, True),
 ])
 def test_layer_wide(backend, fmt, E, K, T, H, I, shared):
-    """objeta_hip_moe_layer_shared_device from 32 tokens: the oracle's routing and
+    """objeta_hip_moe_layer_shared_device at batches: the oracle's routing and
     selected_moe for tokens across the batch, and the per-assignment path for all."""
     experts = make_experts(fmt, E + 1, H, I, H, seed=140 + fmt, gen="gauss")
     table, keep = device_table(backend, fmt, experts[:E])
@@ -98,6 +119,8 @@ def test_layer_wide(backend, fmt, E, K, T, H, I, shared):
     d_ids, d_w = backend.alloc(4 * T * K), backend.alloc(4 * T * K)
     moe = MoeExecutor(backend)
     moe.layer_device(fmt, table, backend.to_device(w_r), None, K, T, d_x, d_x, d_out, d_ids, d_w, H, I, H, shared=sh)
+    if not shared and T * K <= 1024:  # the layer groups from 12 tokens on
+        moe.grouped_device(fmt, table, d_ids, d_w, T, K, d_x, d_x, d_out, H, I, H)
     moe.selected_device(fmt, table, d_ids, d_w, T, K, d_x, d_x, d_ref, H, I, H, shared=sh)
     backend.synchronize()
     assert moe.device_error() == 0
