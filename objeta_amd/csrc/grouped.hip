@@ -847,14 +847,14 @@ bool grouped_supported(int32_t format, uint64_t n_table, uint64_t n_tokens, uint
     return format != OBJETA_HIP_FP4_E2M1;  // split FP4 takes the wide products alone
 }
 
-bool grouped_preferred(int32_t format, uint64_t n_tokens, uint64_t hidden, uint64_t inter, uint64_t out_dim) {
+bool grouped_preferred(int32_t format, uint64_t n_tokens, uint64_t k, uint64_t hidden, uint64_t inter, uint64_t out_dim) {
     if (n_tokens >= kGroupedMinTokens) return true;
     if (n_tokens < 2) return false;
     // bytes per 32 weights of each format
     const uint64_t per32 = format == OBJETA_HIP_Q4_0 ? 18 : format == OBJETA_HIP_Q5_0 ? 22
                          : format == OBJETA_HIP_IQ3_0 ? 14 : 17;
     const uint64_t bytes = (2 * inter * hidden + out_dim * inter) / 32 * per32;
-    return bytes >= kGroupedLargeExpertBytes;
+    return bytes >= kGroupedLargeExpertBytes || (k <= 32 && n_tokens * k * bytes >= kGroupedReadBytes);
 }
 
 int32_t launch_moe_grouped(objeta_hip_context* ctx, int32_t format, hipStream_t s, const objeta_hip_expert_ptrs* table,

@@ -85,10 +85,12 @@ int32_t launch_moe_official_fp4(objeta_hip_context* ctx, hipStream_t s, const ob
                                 uint8_t* inter_values, uint8_t* inter_scales, const OfficialMarks* marks);
 
 // The same layer on the grouped-token products (wide.hip), for batches of at
-// least kOfficialGroupedMinTokens tokens in the grouped path's limits (at the
-// DeepSeek shape the per-token kernels are faster up to 4 tokens, the grouped ones
-// from 6: the per-token path reads the FP8 shared expert once per token).
+// least kOfficialGroupedMinTokens tokens, or 2 where the per-token kernels would read
+// kOfficialGroupedReadBytes, in the grouped path's limits (us, per-token / grouped: hidden
+// 7168, intermediate 2048, top-8 at 2 tokens, 462 MB, 170 / 151, at 4 318 / 187; hidden
+// 2048, intermediate 768, top-4 at 4 tokens, 59 MB, 30 / 41).
 constexpr uint64_t kOfficialGroupedMinTokens = 6;
+constexpr uint64_t kOfficialGroupedReadBytes = uint64_t(256) << 20;
 bool official_grouped_supported(uint64_t n_table, uint64_t n_tokens, uint64_t k, uint64_t hidden, uint64_t inter,
                                 uint64_t out_dim);
 int32_t launch_moe_official_grouped(objeta_hip_context* ctx, hipStream_t s, const objeta_hip_expert_ptrs* table,
@@ -132,8 +134,13 @@ constexpr uint64_t kGroupedMinTokens = 12;
 // per-assignment kernels; the Qwen3-A3B shape's 2.6 MB experts keep the 12-token
 // switch.
 constexpr uint64_t kGroupedLargeExpertBytes = uint64_t(8) << 20;
+// And from 2 tokens when the per-assignment kernels would read this many bytes (us,
+// per-assignment / grouped: Q4_0 2048 x 768, top-8 at 6 tokens, 127 MB, 40 / 44, at 8,
+// 170 MB, 47 / 45, at 10 56 / 52; split FP4 2048 x 768 at 8 tokens, 160 MB, 44 / 45; Q5_0
+// 3072 x 1024, top-4 at 8 tokens, 208 MB, 75 / 50).
+constexpr uint64_t kGroupedReadBytes = uint64_t(128) << 20;
 // Whether the layer entry points run a batch of n_tokens on the grouped path.
-bool grouped_preferred(int32_t format, uint64_t n_tokens, uint64_t hidden, uint64_t inter, uint64_t out_dim);
+bool grouped_preferred(int32_t format, uint64_t n_tokens, uint64_t k, uint64_t hidden, uint64_t inter, uint64_t out_dim);
 // Whether launch_moe_grouped takes this shape.
 bool grouped_supported(int32_t format, uint64_t n_table, uint64_t n_tokens, uint64_t k, uint64_t hidden,
                        uint64_t inter, uint64_t out_dim);

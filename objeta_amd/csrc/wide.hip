@@ -797,8 +797,12 @@ int32_t launch_moe_wide(objeta_hip_context* ctx, int32_t format, hipStream_t s, 
 
 bool official_grouped_supported(uint64_t n_table, uint64_t n_tokens, uint64_t k, uint64_t hidden, uint64_t inter,
                                 uint64_t out_dim) {
-    return n_tokens >= kOfficialGroupedMinTokens && wide_shape(OBJETA_HIP_FP4_E2M1, n_table, k, hidden, inter, out_dim) &&
-           matrices_fit(OBJETA_HIP_FP4_E2M1, true, hidden, inter, out_dim) && n_tokens <= launch_tokens(k, hidden, inter);
+    if (n_tokens < 2 || !wide_shape(OBJETA_HIP_FP4_E2M1, n_table, k, hidden, inter, out_dim)) return false;
+    const uint64_t matrices = 2 * inter * hidden + out_dim * inter;  // an expert's weights
+    if (n_tokens < kOfficialGroupedMinTokens &&
+        n_tokens * (k * (matrices / 32 * 17) + matrices) < kOfficialGroupedReadBytes)
+        return false;
+    return matrices_fit(OBJETA_HIP_FP4_E2M1, true, hidden, inter, out_dim) && n_tokens <= launch_tokens(k, hidden, inter);
 }
 
 // The official layer of launch_moe_official_fp4 on the grouped products: x is quantized
