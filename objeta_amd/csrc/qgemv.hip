@@ -165,8 +165,10 @@ hipError_t launch_generic(hipStream_t s, const uint8_t* q, const float* x, float
     return hipGetLastError();
 }
 
+// Vectors per launch. Three in one launch instead of two and one: Q5_0 5003 x 2880
+// 14.0 -> 10.5 us (a second launch and a second pass over the weights).
 int max_nt_for_lds(size_t per_token, size_t limit, uint64_t remaining) {
-    for (int nt : {8, 4, 2, 1})
+    for (int nt : {8, 4, 3, 2, 1})
         if (static_cast<uint64_t>(nt) <= remaining && per_token * nt <= limit) return nt;
     return 0;
 }
@@ -212,6 +214,7 @@ int32_t launch_qgemv(objeta_hip_context* ctx, int32_t format, hipStream_t s, con
         switch (nt) {                                                                            \
             case 8: e = launch_stream<QRows<F>, 8>(ctx, s, rm, xb, yb, r, c, lpr, lds); break;   \
             case 4: e = launch_stream<QRows<F>, 4>(ctx, s, rm, xb, yb, r, c, lpr, lds); break;   \
+            case 3: e = launch_stream<QRows<F>, 3>(ctx, s, rm, xb, yb, r, c, lpr, lds); break;   \
             case 2: e = launch_stream<QRows<F>, 2>(ctx, s, rm, xb, yb, r, c, lpr, lds); break;   \
             default: e = launch_stream<QRows<F>, 1>(ctx, s, rm, xb, yb, r, c, lpr, lds); break;  \
         }                                                                                        \
@@ -270,6 +273,7 @@ int32_t launch_fp4_split(objeta_hip_context* ctx, hipStream_t s, const void* d_w
             switch (nt) {
                 case 8: e = launch_stream<Fp4Rows, 8>(ctx, s, rm, xb, yb, r, c, lpr, lds); break;
                 case 4: e = launch_stream<Fp4Rows, 4>(ctx, s, rm, xb, yb, r, c, lpr, lds); break;
+                case 3: e = launch_stream<Fp4Rows, 3>(ctx, s, rm, xb, yb, r, c, lpr, lds); break;
                 case 2: e = launch_stream<Fp4Rows, 2>(ctx, s, rm, xb, yb, r, c, lpr, lds); break;
                 default: e = launch_stream<Fp4Rows, 1>(ctx, s, rm, xb, yb, r, c, lpr, lds); break;
             }
@@ -317,6 +321,7 @@ int32_t launch_fp8_rows(objeta_hip_context* ctx, hipStream_t s, const void* d_w,
         switch (nt) {
             case 8: e = launch_stream<Fp8Rows, 8>(ctx, s, rm, xb, yb, r, c, lpr, lds); break;
             case 4: e = launch_stream<Fp8Rows, 4>(ctx, s, rm, xb, yb, r, c, lpr, lds); break;
+            case 3: e = launch_stream<Fp8Rows, 3>(ctx, s, rm, xb, yb, r, c, lpr, lds); break;
             case 2: e = launch_stream<Fp8Rows, 2>(ctx, s, rm, xb, yb, r, c, lpr, lds); break;
             default: e = launch_stream<Fp8Rows, 1>(ctx, s, rm, xb, yb, r, c, lpr, lds); break;
         }
