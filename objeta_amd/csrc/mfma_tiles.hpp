@@ -82,39 +82,57 @@ __device__ __forceinline__ half8 pack8(h2 a, h2 b, h2 c, h2 d) {
     return r;
 }
 
-// nibble dword n (weights 2m, 2m+1 in byte m), optional 5th bits m8 (bit i: weight i)
+// The constants of the decodes that v_and_or_b32 takes from a register: an instruction of
+// gfx9 reads one scalar constant, so mask and magic together cost a separate and and or
+// unless one sits in a vector register (the empty asm hides its value; without side
+// effects, it is hoisted out of the loops).
+__device__ __forceinline__ uint32_t in_vgpr(uint32_t v) {
+    asm("" : "+v"(v));
+    return v;
+}
+
+// nibble dword n (weights 2m, 2m+1 in byte m), optional 5th bits m8 (bit i: weight i):
+// fp16 1024 + q (or 1024 + 16 q) by OR-ing the field into the significand, then the zero
+// point taken off. The 5th bits of a pair go 16 apart, then to above their nibble. (The
+// products by constants that spread them before are multiplies at a quarter of the rate.) The
+// 512-token Q4_0 layer of 128 2048 x 768 experts: 361 -> 353 us.
 template <bool Q5>
 __device__ __forceinline__ half8 nibbles_to_b(uint32_t n, uint32_t m8) {
-    const uint32_t magic = 0x64006400u;
+    const uint32_t magic = in_vgpr(0x64006400u);
     const uint32_t n8 = n >> 8;
     const _Float16 blo = Q5 ? (_Float16)1040.0f : (_Float16)1032.0f;  // 1024 + zero point
     const _Float16 bhi = Q5 ? (_Float16)-80.0f : (_Float16)-72.0f;    // 64 + zero point
     const h2 klo = {blo, blo}, khi = {bhi, bhi}, k16 = {(_Float16)0.0625f, (_Float16)0.0625f};
-    uint32_t sa = 0, sb = 0, sc = 0, sd = 0;
+    uint32_t a = (n & 0x000F000Fu) | magic, b = (n & 0x00F000F0u) | magic;
+    uint32_t c = (n8 & 0x000F000Fu) | magic, d = (n8 & 0x00F000F0u) | magic;
     if constexpr (Q5) {
-        sa = ((m8 & 0x11u) * 0x10010u) & 0x00100010u;
-        sb = ((m8 & 0x22u) * 0x80080u) & 0x01000100u;
-        sc = ((m8 & 0x44u) * 0x04004u) & 0x00100010u;
-        sd = ((m8 & 0x88u) * 0x20020u) & 0x01000100u;
+        const uint32_t h = m8 | (m8 << 12);  // bit i: weight i, bit 16 + i: weight i + 4 (i < 4)
+        a |= (h << 4) & 0x00100010u;
+        b |= (h << 7) & 0x01000100u;
+        c |= (h << 2) & 0x00100010u;
+        d |= (h << 5) & 0x01000100u;
     }
-    const h2 a = as_h2((n & 0x000F000Fu) | sa | magic) - klo;
-    const h2 b = as_h2((n & 0x00F000F0u) | sb | magic) * k16 + khi;
-    const h2 c = as_h2((n8 & 0x000F000Fu) | sc | magic) - klo;
-    const h2 d = as_h2((n8 & 0x00F000F0u) | sd | magic) * k16 + khi;
-    return pack8(a, b, c, d);
+    return pack8(as_h2(a) - klo, as_h2(b) * k16 + khi, as_h2(c) - klo, as_h2(d) * k16 + khi);
 }
 
 // IQ3_0: 2-bit lows lo16 (weights 8kg .. 8kg+7) and 1-bit highs h8 -> the 8 weights
-// q - 4 as exact fp16 in the (w0,w4),(w1,w5),.. order.
+// q - 4 as exact fp16 in the (w0,w4),(w1,w5),.. order: the lows' bytes and the highs'
+// nibbles go 16 apart, a pair's fields stay where they are (q 4^i, exact in the
+// significand) and the zero point's multiply-add scales them back. 19 operations instead
+// of 40 (8 vectors by 14336 x 4096 21.0 -> 18.0 us, 64 vectors 56.7 -> 52.2).
 __device__ __forceinline__ half8 iq3_to_b(uint32_t lo16, uint32_t h8) {
-    const h2 k4 = {(_Float16)1028.0f, (_Float16)1028.0f};
+    const uint32_t magic = in_vgpr(0x64006400u);
+    const uint32_t e = __builtin_amdgcn_perm(0u, lo16, 0x0C010C00u);  // bytes: lows 0..3, 0, lows 4..7, 0
+    const uint32_t h = h8 | (h8 << 12);  // bit i: weight i, bit 16 + i: weight i + 4 (i < 4)
+    const h2 k0 = {(_Float16)1028.0f, (_Float16)1028.0f};
     h2 p[4];
+    p[0] = as_h2(((e & 0x00030003u) | magic) | ((h << 2) & 0x00040004u)) - k0;
+    const _Float16 sc[4] = {(_Float16)1.0f, (_Float16)0.25f, (_Float16)0.0625f, (_Float16)0.015625f};
+    const _Float16 zp[4] = {(_Float16)-1028.0f, (_Float16)-260.0f, (_Float16)-68.0f, (_Float16)-20.0f};
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {  // weights i and i + 4
-        const uint32_t t = (lo16 >> (2 * i)) & 0x303u;
-        const uint32_t hh = (h8 >> i) & 0x11u;
-        const uint32_t v = (t & 3u) | ((t & 0x300u) << 8) | ((hh & 1u) << 2) | ((hh & 0x10u) << 14);
-        p[i] = as_h2(v | 0x64006400u) - k4;
+    for (int i = 1; i < 4; ++i) {
+        const uint32_t v = ((e & (0x00030003u << (2 * i))) | magic) | ((h << (i + 2)) & (0x00040004u << (2 * i)));
+        p[i] = as_h2(v) * h2{sc[i], sc[i]} + h2{zp[i], zp[i]};
     }
     return pack8(p[0], p[1], p[2], p[3]);
 }
@@ -151,11 +169,14 @@ struct Tile<QRows<F>> {
                                                 float& scale) {
         const uint8_t* blk = w + b * kBB;
         auto u16 = [&](uint32_t o) { return static_cast<uint32_t>(*reinterpret_cast<const uint16_t*>(blk + o)); };
+        // a dword at 2-byte alignment as two reads (one unaligned LDS read took 14% longer
+        // over the whole product, two aligned dwords and a byte shift 1 to 3%)
+        auto u32 = [&](uint32_t o) { return u16(o) | (u16(o + 2) << 16); };
         scale = f16_to_f32(u16(0));
         if constexpr (F == kQ4) {
-            return nibbles_to_b<false>(u16(2 + 4 * kg) | (u16(4 + 4 * kg) << 16), 0);
+            return nibbles_to_b<false>(u32(2 + 4 * kg), 0);
         } else if constexpr (F == kQ5) {
-            return nibbles_to_b<true>(u16(6 + 4 * kg) | (u16(8 + 4 * kg) << 16), blk[2 + kg]);
+            return nibbles_to_b<true>(u32(6 + 4 * kg), blk[2 + kg]);
         } else {
             return iq3_to_b(u16(2 + 2 * kg), blk[10 + kg]);
         }
