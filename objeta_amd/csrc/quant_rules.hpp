@@ -45,12 +45,13 @@ OBJ_HD uint16_t f32_to_f16_bits(float value) {
 
 // `(v).round().clamp(0.0, hi) as u8` in Rust: round half away from zero, NaN
 // survives clamp, the saturating cast maps NaN to 0.
+// Negative values round to at most -0 and clamp to 0, so what is left is the rounding of
+// v >= 0 (t = trunc v, v - t exact).
 OBJ_HD uint8_t round_clamp_u8(float v, float hi) {
-    float r = __builtin_roundf(v);
-    if (r != r) return 0;
-    if (r < 0.0f) r = 0.0f;
-    if (r > hi) r = hi;
-    return static_cast<uint8_t>(r);
+    v = __builtin_fmaxf(v, 0.0f);  // NaN -> 0
+    const float t = __builtin_truncf(v);
+    const float r = v - t >= 0.5f ? t + 1.0f : t;
+    return static_cast<uint8_t>(__builtin_fminf(r, hi));
 }
 
 // IEEE division, correctly rounded on host and device alike.
@@ -61,6 +62,31 @@ OBJ_HD float div_rn(float a, float b) {
     return a / b;
 #endif
 }
+
+// Quotients by one divisor: with r = 1/b correctly rounded and q within an ulp of a/b,
+// q + (a - q b) r rounded once is the correctly rounded quotient (Markstein, IBM J. Res.
+// Dev. 34, 1990), three operations instead of a division's ten. Divisors outside
+// [2^-96, 2^96] (where a product could leave the normal range; |a / b| <= 16 here, and a
+// quotient small enough to underflow rounds to the zero point either way) are divided.
+// 4096 x 14336 on the device, us: Q4_0 72 -> 41, Q5_0 312 -> 46, IQ3_0 134 -> 39 (with the
+// rounding below eight operations less and the bit fields gathered in registers).
+struct Quotient {
+    float b, r;
+    bool divide;
+    OBJ_HD explicit Quotient(float divisor) : b(divisor), r(div_rn(1.0f, divisor)) {
+        const uint32_t e = f2u(divisor) >> 23;  // the sign counts as out of range
+        divide = e < 127u - 96u || e > 127u + 96u;
+    }
+    OBJ_HD float operator()(float a) const {
+#if defined(__HIP_DEVICE_COMPILE__)
+        if (!divide) {
+            const float q = a * r;
+            return __builtin_fmaf(__builtin_fmaf(-q, b, a), r, q);
+        }
+#endif
+        return div_rn(a, b);
+    }
+};
 
 // ceil(log2f(y)) as the reference evaluates it (glibc log2f, which is correctly
 // rounded on these inputs), for finite y > 0, in integers: the exact ceiling,
@@ -122,11 +148,17 @@ OBJ_HD uint8_t fp4_scale_raw(float amax) {
 // decode_f8_e8m0 (quant.rs:886-892)
 OBJ_HD float decode_e8m0(uint32_t raw) { return raw == 0 ? u2f(1u << 22) : u2f(raw << 23); }
 
-// quantize_val (quant.rs:894-906): first minimum over the 16-entry table.
-OBJ_HD uint8_t fp4_quantize_val(float val, float scale) {
+// quantize_val (quant.rs:894-906): first minimum over the 16-entry table. Up to
+// magnitude 8 that is the number of midpoints passed (a midpoint itself goes to the lower
+// entry, -0 to entry 0; FP4 4096 x 14336 122 -> 46 us); beyond, and for NaN, the differences round and the table decides.
+OBJ_HD uint8_t fp4_quantize_scaled(float scaled) {
+    const float m = __builtin_fabsf(scaled);
+    if (m <= 8.0f) {
+        const uint32_t i = (m > 0.25f) + (m > 0.75f) + (m > 1.25f) + (m > 1.75f) + (m > 2.5f) + (m > 3.5f) + (m > 5.0f);
+        return static_cast<uint8_t>(i && scaled < 0.0f ? i + 8u : i);
+    }
     const float table[16] = {0.0f, 0.5f, 1.0f, 1.5f, 2.0f, 3.0f, 4.0f, 6.0f,
                              -0.0f, -0.5f, -1.0f, -1.5f, -2.0f, -3.0f, -4.0f, -6.0f};
-    const float scaled = div_rn(val, scale);
     int best = 0;
     float min_diff = __builtin_inff();
     for (int q = 0; q < 16; ++q) {
@@ -149,9 +181,11 @@ OBJ_HD void q4_block(const float* src, uint8_t* dst) {
     const uint16_t h = f32_to_f16_bits(scale);
     dst[0] = static_cast<uint8_t>(h & 0xFF);
     dst[1] = static_cast<uint8_t>(h >> 8);
+    const Quotient by(scale);
+#pragma unroll
     for (int i = 0; i < 16; ++i) {
-        const uint8_t q0 = round_clamp_u8(div_rn(src[2 * i], scale) + 8.0f, 15.0f);
-        const uint8_t q1 = round_clamp_u8(div_rn(src[2 * i + 1], scale) + 8.0f, 15.0f);
+        const uint8_t q0 = round_clamp_u8(by(src[2 * i]) + 8.0f, 15.0f);
+        const uint8_t q1 = round_clamp_u8(by(src[2 * i + 1]) + 8.0f, 15.0f);
         dst[2 + i] = static_cast<uint8_t>(q0 | (q1 << 4));
     }
 }
@@ -160,40 +194,53 @@ OBJ_HD void q5_block(const float* src, uint8_t* dst) {
     const float amax = block_amax(src);
     const float scale = amax > 0.0f ? div_rn(amax, 15.0f) : 1.0e-10f;
     const uint16_t h = f32_to_f16_bits(scale);
-    uint8_t out[22] = {};
-    out[0] = static_cast<uint8_t>(h & 0xFF);
-    out[1] = static_cast<uint8_t>(h >> 8);
-    for (int i = 0; i < 32; ++i) {
-        const uint8_t q = round_clamp_u8(div_rn(src[i], scale) + 16.0f, 31.0f);
-        const uint8_t low = q & 0x0F, high = (q >> 4) & 1;
-        out[6 + i / 2] |= static_cast<uint8_t>((i & 1) ? (low << 4) : low);
-        if (high) out[2 + i / 8] |= static_cast<uint8_t>(1u << (i % 8));
+    dst[0] = static_cast<uint8_t>(h & 0xFF);
+    dst[1] = static_cast<uint8_t>(h >> 8);
+    const Quotient by(scale);
+    uint32_t high = 0;  // bit i: bit 4 of weight i
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+        const uint32_t q0 = round_clamp_u8(by(src[2 * i]) + 16.0f, 31.0f);
+        const uint32_t q1 = round_clamp_u8(by(src[2 * i + 1]) + 16.0f, 31.0f);
+        dst[6 + i] = static_cast<uint8_t>((q0 & 15u) | (q1 << 4));
+        high |= ((q0 >> 4) | ((q1 >> 4) << 1)) << (2 * i);
     }
-    for (int i = 0; i < 22; ++i) dst[i] = out[i];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) dst[2 + i] = static_cast<uint8_t>(high >> (8 * i));
 }
 
 OBJ_HD void iq3_block(const float* src, uint8_t* dst) {
     const float amax = block_amax(src);
     const float scale = amax > 0.0f ? div_rn(amax, 4.0f) : 1.0e-10f;
     const uint16_t h = f32_to_f16_bits(scale);
-    uint8_t out[14] = {};
-    out[0] = static_cast<uint8_t>(h & 0xFF);
-    out[1] = static_cast<uint8_t>(h >> 8);
-    for (int i = 0; i < 32; ++i) {
-        const uint8_t q = round_clamp_u8(div_rn(src[i], scale) + 4.0f, 7.0f);
-        out[2 + i / 4] |= static_cast<uint8_t>((q & 3) << (2 * (i % 4)));
-        out[10 + i / 8] |= static_cast<uint8_t>(((q >> 2) & 1) << (i % 8));
+    dst[0] = static_cast<uint8_t>(h & 0xFF);
+    dst[1] = static_cast<uint8_t>(h >> 8);
+    const Quotient by(scale);
+    uint32_t high = 0;  // bit i: bit 2 of weight i
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+        uint32_t low = 0;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const uint32_t q = round_clamp_u8(by(src[4 * i + j]) + 4.0f, 7.0f);
+            low |= (q & 3u) << (2 * j);
+            high |= (q >> 2) << (4 * i + j);
+        }
+        dst[2 + i] = static_cast<uint8_t>(low);
     }
-    for (int i = 0; i < 14; ++i) dst[i] = out[i];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) dst[10 + i] = static_cast<uint8_t>(high >> (8 * i));
 }
 
 OBJ_HD void fp4_block(const float* src, uint8_t* dst) {
     const uint8_t raw = fp4_scale_raw(block_amax(src));
     dst[0] = raw;
     const float s = decode_e8m0(raw);
+    const Quotient by(s);
+#pragma unroll
     for (int i = 0; i < 16; ++i) {
-        const uint8_t q0 = fp4_quantize_val(src[2 * i], s);
-        const uint8_t q1 = fp4_quantize_val(src[2 * i + 1], s);
+        const uint8_t q0 = fp4_quantize_scaled(by(src[2 * i]));
+        const uint8_t q1 = fp4_quantize_scaled(by(src[2 * i + 1]));
         dst[1 + i] = static_cast<uint8_t>(q0 | (q1 << 4));
     }
 }

@@ -37,6 +37,51 @@ def test_device_quantizer_bytes_equal_cpu(quant, fmt, rows, cols, seed):
     assert np.array_equal(got, orc.quantize_matrix(fmt, m, rows, cols))
 
 
+@pytest.mark.parametrize("fmt", [0, 1, 2, 3])
+@pytest.mark.parametrize("rows,cols,shift", [(1, 32, 0), (3, 672, 0), (5, 416, 0), (67, 160, 0), (67, 160, 2), (67, 160, 4)])
+def test_device_quantizer_ragged_blocks_and_alignment(backend, fmt, rows, cols, shift):
+    """Block counts around a wave's 64 (1, 63, 65) and a ragged last workgroup (335), outputs
+    at 2- and 4-byte alignment, with nothing written past them."""
+    m = orc.gauss(rows * cols, 5 + rows, 0.02)
+    want = orc.quantize_matrix(fmt, m, rows, cols)
+    d_m, d_out = backend.to_device(m), backend.to_device(np.full(len(want) + 16, 0xA5, np.uint8))
+    check(backend.L.objeta_hip_quantize_matrix_device(backend.ctx, fmt, None, d_m.addr(), rows, cols,
+                                                      C.c_void_p(d_out.addr().value + shift)))
+    backend.synchronize()
+    got = d_out.download(np.uint8, len(want) + 16)
+    assert np.array_equal(got[shift:shift + len(want)], want)
+    assert np.all(got[:shift] == 0xA5) and np.all(got[shift + len(want):] == 0xA5)
+
+
+@pytest.mark.parametrize("fmt", [0, 1, 2, 3])
+def test_device_quantizer_rounding_edges(quant, fmt):
+    """Values a unit in the last place around every rounding boundary of a block's codes,
+    both signs, with block maxima from subnormal to 2^127 (both sides of the range where
+    quotients come from a reciprocal), maxima with all-ones significands among them."""
+    div = {0: 7.0, 1: 15.0, 2: 4.0, 3: 6.0}[fmt]
+    mids = np.array([0.25, 0.75, 1.25, 1.75, 2.5, 3.5, 5.0, 0.0] if fmt == 3 else np.arange(0, div, div / 8) // 1 + 0.5)
+    rng = np.random.default_rng(fmt)
+    blocks = []
+    for e in (-148, -140, -126, -100, -97, -96, -95, -60, -20, 0, 3, 40, 94, 95, 96, 97, 98, 110, 126):
+        for frac in (1.0, 2.0 - 2.0 ** -23, 1.0 + rng.random(), 1.0 + rng.random()):
+            amax = np.float32(min(np.ldexp(frac, e), 3e38))
+            step = np.float64(np.float32(np.float64(amax) / div)) if fmt != 3 else 2.0 ** np.ceil(
+                np.log2(max(float(amax) / 6.0, 2.0 ** -127)))
+            b = np.zeros(32, np.float64)
+            b[:8], b[8:16], b[16:24] = mids[:8] * step, -mids[:8] * step, mids[:8] * step
+            v = b.astype(np.float32)
+            v[0:24:3] = np.nextafter(v[0:24:3], np.float32(np.inf))
+            v[1:24:3] = np.nextafter(v[1:24:3], np.float32(-np.inf))
+            v[24:31] = rng.standard_normal(7).astype(np.float32) * np.float32(amax / 3)
+            v = np.clip(v, -amax, amax)
+            v[31] = amax
+            blocks.append(v)
+    m = np.concatenate(blocks).astype(np.float32)
+    rows = len(blocks)
+    got = quant.quantize_matrix(QuantFormat(fmt), m, QGemvShape.new(QuantFormat(fmt), rows, 32))
+    assert np.array_equal(got, orc.quantize_matrix(fmt, m, rows, 32))
+
+
 @pytest.mark.parametrize("seed", [0, 42])
 def test_device_quantizer_reference_lcg_data(quant, seed):
     # the reference's own test data recipe (seeded_f32s, quant.rs:1610-1662)
