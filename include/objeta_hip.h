@@ -344,12 +344,10 @@ int32_t objeta_hip_moe_down_device(objeta_hip_context* ctx, int32_t format, obje
  * d_router_w [n_experts][hidden] (+ d_router_bias) writes d_ids_out/d_weights_out
  * [n_tokens][k], then the selected experts of d_table (n_experts entries) run:
  * below 12 tokens on the per-assignment kernels of objeta_hip_moe_selected_device,
- * from 12 tokens on the grouped-token products of objeta_hip_moe_grouped_device
- * whenever that path takes the shape (on MI355X at hidden 2048, 128 experts,
- * top-8 the per-assignment kernels are faster up to 10 tokens, the two are even at
- * 12 and the grouped ones faster from 14 on). When one expert's three matrices
- * take 8 MiB or more (hidden 7168, intermediate 2048) the grouped products run
- * from 2 tokens. The two agree within the fp32
+ * from 12 tokens on the grouped-token products of objeta_hip_moe_grouped_device (any
+ * number of tokens) whenever that path takes the shape; from 2 tokens when one expert's
+ * three matrices take 8 MiB or more, or n_tokens * k experts' 128 MiB or more (what the
+ * per-assignment kernels would read). The two agree within the fp32
  * tolerance, not bit for bit. No host
  * synchronisation; graph-capturable. No reference counterpart as one call: the
  * reference routes on the host (deepseek_single_layer_moe.rs:687-743) and then
@@ -571,9 +569,10 @@ int32_t objeta_hip_fp8_act_fp8_weight_gemv_device(objeta_hip_context* ctx, objet
  * d_inter_scales [n_tokens*kk][intermediate/128] (nullable; kk = k + 1 with a
  * shared expert, else k) receive the intermediates' FP8 codes: rows t*k + j for
  * the routed slots, then n_tokens*k + t for the shared expert. From 6 tokens
- * (and up to 1024 (token, slot) assignments over at most 1024 experts) the layer
- * runs on the grouped-token products of objeta_hip_moe_grouped_device: each selected
- * expert, and the shared expert, read once per set of up to 8 of its tokens. The
+ * (2 where the per-token kernels would read 256 MiB or more of expert weights; up to 4096
+ * (token, slot) assignments over at most 1024 experts) the layer runs on the
+ * grouped-token products of objeta_hip_moe_grouped_device: each selected expert, and the
+ * shared expert, read once per set of up to 16 of its tokens. The
  * results agree with the per-token kernels within the fp32 tolerance (the sums run
  * in another order), so an intermediate code near a rounding boundary can differ. */
 int32_t objeta_hip_moe_official_fp4_device(objeta_hip_context* ctx, objeta_hip_stream stream,
@@ -711,7 +710,7 @@ typedef struct {
  * host, the cache resolving the union of the batch's selected experts (get, then
  * insert with a copy on the copy stream for misses: the reference's admission and
  * counters), and the expert kernels waiting for that layer's copies only; batches
- * of 12 tokens and more run the grouped-token products. prefetch_next != 0 also
+ * run the grouped-token products where objeta_hip_moe_layer_device would. prefetch_next != 0 also
  * evaluates layer l+1's router on layer l's input and starts copying its predicted
  * experts' absent tensors behind layer l's own (objeta_hip_cache_prefetch).
  * ids_out / weights_out (host, [n_layers][n_tokens][k], nullable) receive the

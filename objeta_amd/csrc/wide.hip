@@ -7,29 +7,29 @@
 // split_row), weights are exact in fp16, and the row's block scale multiplies the sum of
 // a 32-column block in fp32.
 //
-// Work split: a workgroup takes 128 weight rows (gate/up: 64 of each matrix) and a work
-// item of 32 vectors (16 for split FP4), and walks the columns in chunks of 128. Its four
+// Work split: a workgroup takes 64 or 128 weight rows (gate/up: half of each matrix) and
+// a work item of 16 or 32 vectors, and walks the columns in chunks (Work, below). Its four
 // waves are two row halves times two halves of the chunk's blocks, so one A operand read
-// from LDS serves four row tiles and a weight is decoded once per work item. The next
-// chunk's loads travel in registers during the products.
+// from LDS serves all row tiles of a wave and a weight is decoded once per work item. The
+// next chunk's loads travel in registers during the products.
 //
-// What bounds it: latency. At 512 tokens of hidden 2048, intermediate 768, 128 experts,
-// top-8 (Q4_0) the matrix cores are about a quarter busy and the VALU (decode, two
-// operations per output of a block) a third; three workgroups per CU hide the rest best:
-//   64 vectors per work item, two workgroups per CU: 476 us for the layer; 32 vectors,
-//   three: 366; 32 vectors in 128 registers (four per CU, 100 bytes of spills): 663.
-// The per-assignment kernels took 1893 us for that layer, the eight-member sets of
-// grouped.hip 188 us for the 97-token Q5_0 layer that takes 126 here, and eight passes
-// of gemv_mfma_kernel 73 us for 64 vectors by 4096 x 4096 (Q4_0; 25.6 here).
+// What bounds it: with few vectors per expert the weights' loads in flight (3.1 to 3.4
+// TB/s); with many, latency and the LDS reads. At 512 tokens of hidden 2048, intermediate
+// 768, 128 experts, top-8 (Q4_0) the matrix cores are about a quarter busy and the VALU a
+// third. Layer times there by shape (vectors, rows, columns of a chunk; workgroups per CU):
+// 64, 128, 128; 2: 476 us. 32, 128, 128; 3: 353 (in 128 registers, 100 bytes of spills: 663).
+// 32, 64, 256; 4: 440. 32, 64, 128; 5: 570. 32, 256, 128; 2: 419. 32, 128, 256; 2: 388. 16, 64,
+// 256; 4: 376. Before: the per-assignment kernels 1893 us; sets of eight 188 us for the
+// 97-token Q5_0 layer that takes 123 here; eight passes of gemv_mfma_kernel 73 us for 64
+// vectors by 4096 x 4096 (Q4_0; 24.6 here).
 //
 // Rounding (relative to 64-bit results, against the kernels before): a running sum over
-// two chunks, added to a total, keeps the chains short. The two parts' block sums are
-// added in fp32: taking both through one MFMA accumulator costs less but the unit
-// truncates (5.1e-8 per block instead of 2.6e-8, with the low part first biased by
+// 256 columns (split FP4: 512), added to a total, keeps the chains short. The two parts'
+// block sums are added in fp32: taking both through one MFMA accumulator costs less but the
+// unit truncates (5.1e-8 per block instead of 2.6e-8, with the low part first biased by
 // 7e-9, which adds up over the blocks). Split FP4 keeps the parts' sums apart (its scales
-// are powers of two, so the high parts' sums are nearly exact), which takes the registers
-// of a second vector tile. GEMV at 64 vectors 9.4e-8 (before: 1.06e-7), the 512-token
-// layer 1.92e-7 (2.13e-7).
+// are powers of two, so the high parts' sums are nearly exact). GEMV at 64 vectors 9.4e-8
+// (before: 1.06e-7), the 512-token layer 1.92e-7 (2.13e-7).
 #include "mfma_tiles.hpp"
 
 namespace objeta {
