@@ -30,8 +30,8 @@
 // hardware conversion's pairs) and FP8 weights come in element order, and so do
 // their split activations.
 //
-// The experts' sets of 8 take the block formats up to 8 tokens; split FP4 and larger
-// batches run in wide.hip.
+// The sets of 8 take the block formats up to 8 tokens and any format's batches of few
+// assignments (few_assignments); the others run in wide.hip.
 //
 // MFMA roles (D = A B, 16x16x32): A = activation parts, row m = 2 * token + part
 // (8 tokens per instruction); B = weights, column n = output row. Lane l holds
@@ -295,11 +295,24 @@ __device__ __forceinline__ void slab_store4(uint32_t* lds, uint32_t seg, const u
         }
     }
 }
+// FP4 scale rows (seg <= 16 dwords): one dword per thread, thread t row t / 16.
+__device__ __forceinline__ void scale_load(const uint8_t* base, size_t pitch, uint32_t r0, uint32_t rows, uint32_t seg,
+                                           uint32_t& v) {
+    const uint32_t rr = threadIdx.x >> 4, c = threadIdx.x & 15;
+    const uint32_t r = r0 + rr < rows ? r0 + rr : rows - 1;
+    if (c < seg) v = as_global(reinterpret_cast<const uint32_t*>(base + static_cast<size_t>(r) * pitch))[c];
+}
+__device__ __forceinline__ void scale_store(uint32_t* lds, uint32_t stride, uint32_t seg, uint32_t v) {
+    const uint32_t rr = threadIdx.x >> 4, c = threadIdx.x & 15;
+    if (c < seg) lds[rr * stride + c] = v;
+}
+
 // One chunk's staged bytes of every matrix of the workgroup, in registers.
 template <class R, int M, uint32_t CH>
 struct Staged {
     static constexpr uint32_t kSeg = Tile<R>::wdw(CH);
     u32x4 w[M][SlabUnits<kSeg>::kN];
+    uint32_t s[M];  // FP4 scales: CH / 128 <= 16 dwords per row
 };
 
 // grid = (ceil(rows / 16), gy), 256 threads; workgroup (x, y) takes member sets y,
@@ -320,7 +333,9 @@ __global__ __launch_bounds__(256) void moe_grouped_kernel(GroupWs gw, const _Flo
     constexpr int kB = kChunk / 32 / 4;  // blocks per wave and chunk
     constexpr uint32_t kSeg = Tile<R>::wdw(kChunk);           // weight dwords per row of a full chunk
     constexpr uint32_t kWStride = SlabUnits<kSeg>::kStride;    // LDS dwords per staged weight row
-    static_assert(Tile<R>::lds_dw(kChunk) == kSlab * kWStride, "LDS chunk layout");
+    constexpr uint32_t kSStride = Tile<R>::sdw(kChunk) + 1;    // LDS dwords per staged scale row (FP4)
+    static_assert(Tile<R>::lds_dw(kChunk) == kSlab * kWStride + (Tile<R>::kScales ? kSlab * kSStride : 0u),
+                  "LDS chunk layout");
     const uint32_t n_sets = gw.hdr[1];
     const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const uint32_t r0 = blockIdx.x * kSlab;
@@ -340,7 +355,7 @@ __global__ __launch_bounds__(256) void moe_grouped_kernel(GroupWs gw, const _Flo
         R mt[kMats];
         mt[0] = GATEUP ? RowsOf<R>::make(P.gate, P.gate_scale, cols) : RowsOf<R>::make(P.down, P.down_scale, cols);
         if constexpr (GATEUP) mt[kMats - 1] = RowsOf<R>::make(P.up, P.up_scale, cols);
-        const size_t wpitch = Tile<R>::wpitch(mt[0]);
+        const size_t wpitch = Tile<R>::wpitch(mt[0]), spitch = Tile<R>::spitch(mt[0]);
         SlabLanes<kSeg> lanes;
         lanes.init(r0, rows, wpitch);
         __amdgpu_buffer_rsrc_t rs[kMats];
@@ -357,6 +372,8 @@ __global__ __launch_bounds__(256) void moe_grouped_kernel(GroupWs gw, const _Flo
             for (int t = 0; t < kMats; ++t) {
                 slab_load4<kSeg, FULL>(rs[t], static_cast<uint32_t>(Tile<R>::wrow(mt[t], kc0) - Tile<R>::wrow(mt[t], 0)), lanes,
                                  Tile<R>::wdw(kc), st.w[t]);
+                if constexpr (Tile<R>::kScales)
+                    scale_load(Tile<R>::srow(mt[t], kc0), spitch, r0, rows, Tile<R>::sdw(kc), st.s[t]);
             }
         };
         auto operands = [&](uint32_t kc0, half8 (&xr)[kB]) {
@@ -376,6 +393,8 @@ __global__ __launch_bounds__(256) void moe_grouped_kernel(GroupWs gw, const _Flo
             for (int t = 0; t < kMats; ++t) {
                 uint32_t* base = tl + buf * buf_dw + t * Tile<R>::lds_dw(kChunk);
                 slab_store4<kSeg, FULL>(base, Tile<R>::wdw(kc), st.w[t]);
+                if constexpr (Tile<R>::kScales)
+                    scale_store(base + kSlab * kWStride, kSStride, Tile<R>::sdw(kc), st.s[t]);
             }
         };
         f32x4 acc[kMats];
@@ -399,11 +418,12 @@ __global__ __launch_bounds__(256) void moe_grouped_kernel(GroupWs gw, const _Flo
             for (int t = 0; t < kMats; ++t) {
                 const uint32_t* base = tl + (c & 1) * buf_dw + t * Tile<R>::lds_dw(kChunk);
                 const uint8_t* wl = reinterpret_cast<const uint8_t*>(base + (lane & 15) * kWStride);
+                const uint8_t* sl = reinterpret_cast<const uint8_t*>(base + kSlab * kWStride + (lane & 15) * kSStride);
 #pragma unroll
                 for (int i = 0; i < kB; ++i) {
                     if (b0 + static_cast<uint32_t>(i) >= b1) break;
                     float sc;
-                    const half8 bw = Tile<R>::get(wl, nullptr, 0u, b0 + static_cast<uint32_t>(i), kg, sc);
+                    const half8 bw = Tile<R>::get(wl, sl, 0u, b0 + static_cast<uint32_t>(i), kg, sc);
                     const f32x4 z = {0.f, 0.f, 0.f, 0.f};
                     const f32x4 r = __builtin_amdgcn_mfma_f32_16x16x32_f16(xa[i], bw, z, 0, 0, 0);
 #pragma unroll
@@ -836,6 +856,37 @@ int32_t launch_gemv_mfma(objeta_hip_context* ctx, hipStream_t s, int32_t format,
     return 0;
 }
 
+// Whether a batch has so few assignments (token, slot; the shared expert is one more slot)
+// that the sets of eight are the faster form. The wide products make a work item of 64
+// weight rows per expert and walk its columns in one chain with one LDS buffer; with fewer
+// work items than the CUs take at once, that chain is the time. A set of eight takes 16 rows
+// of each matrix with two buffers: more workgroups per expert, until the weights' bytes are
+// the time or experts have more than eight of the tokens (their weights are read again).
+// IQ3_0, the dearest to decode, and split FP4 turn earlier. us per layer, wide products /
+// sets of eight (64 experts, 2048 x 768: 128; Zipf popularity), below | past the line:
+//   Q4_0 4096 x 1536  top-1, 12 tokens 61 / 47, top-2, 24 85 / 83 | top-4, 24 120 / 127
+//   Q4_0 7168 x 2048  top-1, 9 tokens 92 / 74, top-4, 10 177 / 173 | top-4, 12 187 / 188
+//   Q5_0 2048 x 1408  top-1, 12 tokens 49 / 36, top-2, 32 60 / 56 | top-8, 14 84 / 85
+//   IQ3_0 2048 x 768  top-1, 12 tokens 38 / 35, top-2, 16 41 / 40 | top-4, 12 45 / 46
+//   FP4 7168 x 2048   top-1, 2 tokens 80 / 51, top-2, 8 115 / 109 | top-2, 10 121 / 122
+//   FP4 4608 x 1664   top-2, 5 tokens 64 / 56, top-1, 32 92 / 89 | top-4, 12 108 / 114
+//   FP4 4096 x 1408   top-2, 8 tokens 63 / 54, top-8, 4 89 / 80 | top-8, 8 106 / 108
+// The largest losses near the line over 620 such layers: FP4 7168 x 2048 top-8, 2 tokens 122
+// / 132 below, 4096 x 1408 top-4, 12 tokens 93 / 87 past it.
+bool few_assignments(int32_t format, uint64_t n_table, uint64_t n_tokens, uint64_t k, bool shared, uint64_t hidden,
+                     uint64_t inter, uint64_t out_dim) {
+    if (k == 0 || k > 32 || n_table == 0 || n_table > kGMaxTable || n_tokens > kGMaxAssign) return false;
+    if (hidden > (1u << 20) || inter > (1u << 20) || out_dim > (1u << 20)) return false;
+    // one matrix's weights over all assignments (the limits also keep its offsets in 32 bits)
+    const uint64_t a = n_tokens * (k + (shared ? 1 : 0)), weights = a * inter * (hidden > out_dim ? hidden : out_dim);
+    switch (format) {
+        case OBJETA_HIP_Q4_0:
+        case OBJETA_HIP_Q5_0: return a <= 72 && weights <= 640u << 20;
+        case OBJETA_HIP_IQ3_0: return a <= 40 && weights <= 96u << 20;
+        default: return a <= 40 && weights <= 240u << 20;
+    }
+}
+
 bool grouped_supported(int32_t format, uint64_t n_table, uint64_t n_tokens, uint64_t k, uint64_t hidden,
                        uint64_t inter, uint64_t out_dim) {
     if (format < OBJETA_HIP_Q4_0 || format > OBJETA_HIP_FP4_E2M1) return false;
@@ -844,7 +895,8 @@ bool grouped_supported(int32_t format, uint64_t n_table, uint64_t n_tokens, uint
     if (hidden == 0 || inter == 0 || hidden % 64 || inter % 64 || hidden > (1u << 20) || inter > (1u << 20) ||
         out_dim > (1u << 20))
         return false;
-    return format != OBJETA_HIP_FP4_E2M1;  // split FP4 takes the wide products alone
+    // split FP4 runs on the sets of eight for few assignments alone, which are wide_supported
+    return format != OBJETA_HIP_FP4_E2M1;
 }
 
 bool grouped_preferred(int32_t format, uint64_t n_tokens, uint64_t k, uint64_t hidden, uint64_t inter, uint64_t out_dim) {
@@ -865,7 +917,8 @@ int32_t launch_moe_grouped(objeta_hip_context* ctx, int32_t format, hipStream_t 
     if (format < OBJETA_HIP_Q4_0 || format > OBJETA_HIP_FP4_E2M1)
         OBJ_FAIL(kInvalidInput, action, strf("unknown format %d", format));
     if (n_tokens == 0 || out_dim == 0) return 0;
-    if (wide_supported(format, n_table, n_tokens, k, hidden, inter, out_dim))
+    const bool few = few_assignments(format, n_table, n_tokens, k, shared != nullptr, hidden, inter, out_dim);
+    if (!few && wide_supported(format, n_table, n_tokens, k, hidden, inter, out_dim))
         return launch_moe_wide(ctx, format, s, table, n_table, shared, ids, wts, n_tokens, k, x, resid, out, hidden, inter,
                                out_dim, limit);
     if (k == 0 || k > 32) OBJ_FAIL(kInvalidInput, action, "k must be in 1..=32");
@@ -878,6 +931,7 @@ int32_t launch_moe_grouped(objeta_hip_context* ctx, int32_t format, hipStream_t 
         OBJ_FAIL(kUnsupported, action, "hidden and intermediate must be non-zero multiples of 64 (<= 2^20)");
     if (format == OBJETA_HIP_FP4_E2M1 && (hidden % 128 || inter % 128))
         OBJ_FAIL(kUnsupported, action, "the grouped path takes split-FP4 experts with hidden and intermediate % 128 == 0");
+    if (format == OBJETA_HIP_FP4_E2M1 && !few) OBJ_FAIL(kUnsupported, action, "split-FP4 matrices above 2^31 bytes");
     if (!table || !ids || !wts || !x || !out) OBJ_FAIL(kInvalidInput, action, "NULL device pointer");
     if (reinterpret_cast<uintptr_t>(x) % 16) OBJ_FAIL(kInvalidInput, action, "x must be 16-byte aligned");
     const uint32_t A = static_cast<uint32_t>(n_tokens * k), T = static_cast<uint32_t>(n_tokens);
@@ -910,7 +964,8 @@ int32_t launch_moe_grouped(objeta_hip_context* ctx, int32_t format, hipStream_t 
     float* part = reinterpret_cast<float*>(b + o_part);
     uint32_t* err = ctx->err_word;
     const uint32_t cus = ctx->info.compute_units > 0 ? static_cast<uint32_t>(ctx->info.compute_units) : 256u;
-    const bool perm = Tile<QRows<kQ4>>::kPermuted;  // all block formats
+    // the split order follows the weights' order (element order for FP4)
+    const bool perm = format == OBJETA_HIP_FP4_E2M1 ? Tile<Fp4Rows>::kPermuted : Tile<QRows<kQ4>>::kPermuted;
     hipLaunchKernelGGL(moe_prepare_kernel, dim3(1 + T), dim3(256), 0, s, ids, A, static_cast<uint32_t>(n_table), table,
                        shared, T, gw, err, x, H, xh, xl, xmult, perm ? 1u : 0u);
     hipError_t e;
@@ -928,7 +983,10 @@ int32_t launch_moe_grouped(objeta_hip_context* ctx, int32_t format, hipStream_t 
             e = launch_grouped<QRows<kIQ3>>(s, gw, xh, xl, xmult, act, ah, al, amult, part, A, NR, NS, kk,
                                             H, I, O, limit, cus);
             break;
-        default: OBJ_FAIL(kUnsupported, action, "split-FP4 matrices above 2^31 bytes");
+        default:
+            e = launch_grouped<Fp4Rows>(s, gw, xh, xl, xmult, act, ah, al, amult, part, A, NR, NS, kk, H, I,
+                                        O, limit, cus);
+            break;
     }
     if (e == hipSuccess) {
         launch_moe_combine(s, ids, wts, part, shared ? part + static_cast<size_t>(A) * O : nullptr, resid, out, T, kk, O,

@@ -149,10 +149,14 @@ int32_t launch_moe_grouped(objeta_hip_context* ctx, int32_t format, hipStream_t 
                            const float* x, const float* resid, float* out, uint64_t hidden, uint64_t inter,
                            uint64_t out_dim, float limit);
 
+// Whether launch_moe_grouped takes the sets of eight for the batch where the wide products
+// take it too (measured at the definition).
+bool few_assignments(int32_t format, uint64_t n_table, uint64_t n_tokens, uint64_t k, bool shared, uint64_t hidden,
+                     uint64_t inter, uint64_t out_dim);
 // The same layer on the wide products (wide.hip): work items of up to 16 or 32 tokens of
 // an expert, any number of tokens. Split FP4 takes them at any batch, the block formats
 // from 9 tokens (below, sets of 8 hold every expert's tokens: Q5_0 3072 x 2048 at 3 tokens
-// 57 us on them, 66 here; Q4_0 2048 x 768 at 16 tokens 60 / 57, at 48 104 / 83).
+// 57 us on them, 66 here), all but few_assignments.
 constexpr uint64_t kWideMinTokens = 9;
 bool wide_supported(int32_t format, uint64_t n_table, uint64_t n_tokens, uint64_t k, uint64_t hidden, uint64_t inter,
                     uint64_t out_dim);

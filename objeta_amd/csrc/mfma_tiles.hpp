@@ -139,9 +139,9 @@ __device__ __forceinline__ half8 iq3_to_b(uint32_t lo16, uint32_t h8) {
 
 // ------------------------------------------------------------- staged tiles
 // Staged row segments: weights (and, for the split FP4 layout, the E8M0 scales) of columns
-// [c0, c0 + kc). wdw / sdw: dwords of a row segment. kChunkGU / kChunkDn (block formats):
-// columns per staged chunk of the eight-member sets (grouped.hip), gate and up together /
-// down, the widths that measured fastest there. kTileScale: one E8M0 byte per 128 x 128
+// [c0, c0 + kc). wdw / sdw: dwords of a row segment. kChunkGU / kChunkDn: columns per
+// staged chunk of the eight-member sets (grouped.hip), gate and up together / down, the
+// widths that measured fastest there; lds_dw: LDS dwords of such a chunk. kTileScale: one E8M0 byte per 128 x 128
 // tile (FP8), taken per chunk into a register by tile_scales instead of being staged per
 // row.
 template <class R>
@@ -188,8 +188,12 @@ struct Tile<Fp4Rows> {
     static constexpr bool kPermuted = false;
     static constexpr bool kScales = true;
     static constexpr bool kTileScale = false;
+    static constexpr uint32_t kChunkGU = 512, kChunkDn = 512;
     static constexpr __host__ __device__ uint32_t wdw(uint32_t kc) { return kc / 8; }   // kc / 2 bytes
     static constexpr __host__ __device__ uint32_t sdw(uint32_t kc) { return kc / 128; }  // kc / 32 bytes (kc % 128 == 0)
+    static constexpr __host__ __device__ uint32_t lds_dw(uint32_t kc) {
+        return kSlab * (wdw(kc) + 4) + kSlab * (sdw(kc) + 1);
+    }
     static __device__ __forceinline__ size_t wpitch(const Fp4Rows& m) { return m.wrow; }
     static __device__ __forceinline__ size_t spitch(const Fp4Rows& m) { return m.srow; }
     static __device__ __forceinline__ const uint8_t* wrow(const Fp4Rows& m, uint32_t c0) { return m.w + c0 / 2; }

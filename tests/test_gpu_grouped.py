@@ -257,3 +257,35 @@ def test_layer_one_token_shared_expert_second_down_launch(backend, fmt, K):
     added by a second launch; the token matches the oracle's routing and selected_moe
     with the shared expert."""
     test_layer_batch_runs_grouped_with_shared_expert(backend, fmt, 12, K, 1, 256, 2048, 0.0)
+
+
+@pytest.mark.parametrize("fmt,E,K,T,H,I,O", [
+    (Q4, 5, 3, 2, 1088, 320, 1088),    # two whole chunks and a short one, a chunk and a short one
+    (Q4, 6, 1, 64, 1024, 512, 520),    # whole chunks; groups of more than eight; a last slab of 8 rows
+    (Q5, 4, 2, 5, 1088, 320, 200),
+    (Q5, 9, 8, 9, 1024, 512, 1024),    # 72 assignments: the most that few means for Q4_0 and Q5_0
+    (IQ3, 6, 4, 8, 1088, 320, 1088),
+    (IQ3, 6, 4, 10, 1024, 512, 1024),  # 40
+    (FP4, 3, 2, 1, 1152, 640, 1152),
+    (FP4, 12, 1, 40, 1024, 512, 1032),
+    (FP4, 7, 4, 10, 1152, 640, 1152),
+])
+def test_grouped_sets_of_eight(backend, fmt, E, K, T, H, I, O):
+    """Few assignments: the sets of eight (16 rows per workgroup, two chunk buffers of 512
+    columns for gate and up, 256 for down, split FP4 512) for every format."""
+    test_grouped_matches_oracle_and_per_assignment(backend, fmt, E, K, T, H, I, O)
+
+
+@pytest.mark.parametrize("fmt,E,K,T,H,I", [
+    (Q4, 8, 4, 12, 1088, 320),   # 60 with the shared expert's: sets of eight
+    (Q4, 8, 4, 15, 1088, 320),   # 75: the wide products
+    (Q5, 4, 1, 36, 1024, 512),   # 72; the shared expert's set spans five sets
+    (IQ3, 8, 2, 13, 1088, 320),  # 39
+    (FP4, 8, 2, 13, 1152, 640),  # 39
+    (FP4, 8, 2, 14, 1152, 640),  # 42: wide
+    (Q4, 3, 2, 3, 2112, 2368),   # experts of 8.4 MB: grouped from 2 tokens
+    (Q5, 3, 2, 2, 2112, 1984),
+    (IQ3, 3, 2, 3, 2560, 2560),
+])
+def test_layer_sets_of_eight_with_shared_expert(backend, fmt, E, K, T, H, I):
+    test_layer_batch_runs_grouped_with_shared_expert(backend, fmt, E, K, T, H, I, 0.0)
