@@ -1686,7 +1686,7 @@ extern "C" int32_t objeta_hip_moe_stack_cached(objeta_hip_context* ctx, int32_t 
                 rc = set_error(kDriver, __FILE__, __LINE__, __func__, "stack_table_h2d", hipGetErrorString(e));
                 break;
             }
-            if (grouped_preferred(format, T, k, hidden, intermediate, hidden) &&
+            if (grouped_preferred(format, T, k, false, hidden, intermediate, hidden) &&
                 grouped_supported(format, uni.size(), T, k, hidden, intermediate, hidden)) {
                 rc = launch_moe_grouped(ctx, format, s, d_tab, uni.size(), nullptr, d_rids, d_w, T, k, d_h, d_h, d_h,
                                         hidden, intermediate, hidden, 0.f);

@@ -899,14 +899,27 @@ bool grouped_supported(int32_t format, uint64_t n_table, uint64_t n_tokens, uint
     return format != OBJETA_HIP_FP4_E2M1;
 }
 
-bool grouped_preferred(int32_t format, uint64_t n_tokens, uint64_t k, uint64_t hidden, uint64_t inter, uint64_t out_dim) {
+bool grouped_preferred(int32_t format, uint64_t n_tokens, uint64_t k, bool shared, uint64_t hidden, uint64_t inter,
+                       uint64_t out_dim) {
     if (n_tokens >= kGroupedMinTokens) return true;
     if (n_tokens < 2) return false;
     // bytes per 32 weights of each format
     const uint64_t per32 = format == OBJETA_HIP_Q4_0 ? 18 : format == OBJETA_HIP_Q5_0 ? 22
                          : format == OBJETA_HIP_IQ3_0 ? 14 : 17;
     const uint64_t bytes = (2 * inter * hidden + out_dim * inter) / 32 * per32;
-    return bytes >= kGroupedLargeExpertBytes || (k <= 32 && n_tokens * k * bytes >= kGroupedReadBytes);
+    if (bytes >= kGroupedLargeExpertBytes) return true;
+    if (k > 32) return false;
+    const uint64_t groups = hidden / 64;  // of 64 columns, one to a lane
+    if (inter <= 1024 && groups >= 32 && (groups & (groups - 1)) == 0) {
+        const bool dear = format == OBJETA_HIP_Q5_0 || format == OBJETA_HIP_IQ3_0;
+        if (groups > 64) return false;
+        if (groups == 64) {
+            const uint64_t limit = dear ? kGroupedReadBytesDear4096 : shared ? kGroupedReadBytesShared4096 : kGroupedReadBytes4096;
+            return n_tokens * (k + (shared ? 1 : 0)) * bytes >= limit;
+        }
+        if (!dear && !shared) return n_tokens * k * bytes >= kGroupedReadBytes2048;
+    }
+    return n_tokens * k * bytes >= kGroupedReadBytes;
 }
 
 int32_t launch_moe_grouped(objeta_hip_context* ctx, int32_t format, hipStream_t s, const objeta_hip_expert_ptrs* table,

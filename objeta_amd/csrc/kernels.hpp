@@ -135,12 +135,26 @@ constexpr uint64_t kGroupedMinTokens = 12;
 // switch.
 constexpr uint64_t kGroupedLargeExpertBytes = uint64_t(8) << 20;
 // And from 2 tokens when the per-assignment kernels would read this many bytes (us,
-// per-assignment / grouped: Q4_0 2048 x 768, top-8 at 6 tokens, 127 MB, 40 / 44, at 8,
-// 170 MB, 47 / 45, at 10 56 / 52; split FP4 2048 x 768 at 8 tokens, 160 MB, 44 / 45; Q5_0
-// 3072 x 1024, top-4 at 8 tokens, 208 MB, 75 / 50).
+// per-assignment / grouped: Q5_0 2048 x 1408 top-4 at 6 tokens, 136 MiB, 63 / 46; Q4_0 2560
+// x 1024 top-4 at 8, 135 MiB, 51 / 42; split FP4 3072 x 1408 top-4 at 5, 132 MiB, 63 / 51).
 constexpr uint64_t kGroupedReadBytes = uint64_t(128) << 20;
+// Later where the per-assignment kernels run best, with rows whose 64-column groups fill
+// whole waves (hidden 2048, 4096, 8192) and an intermediate of at most 1024, while the
+// grouped products walk such a row in one chain that grows with hidden: at 8192 not at all
+// below 12 tokens. A shared expert is read once per token by the per-assignment kernels;
+// at 4096 its bytes count. us, per-assignment / grouped:
+//   2048 (cheap formats) Q4_0 2048 x 768 top-8, 8 tokens, 162 MiB, 44 / 46, 10, 203, 53 / 50
+//   4096                 Q4_0 4096 x 1024 top-8, 4, 216 MiB, 59 / 70, top-4, 10, 270, 73 / 70
+//   4096, shared expert  FP4 4096 x 768 top-4, 9, 215 MiB with it, 59 / 62, 11, 263, 67 / 65
+//   4096, Q5_0 and IQ3_0 IQ3_0 4096 x 1024 top-8, 4, 168 MiB, 71 / 82, top-6, 6, 189, 80 / 79
+//   8192                 Q4_0 8192 x 384 top-8, 8, 324 MiB, 85 / 108
+constexpr uint64_t kGroupedReadBytes2048 = uint64_t(168) << 20;
+constexpr uint64_t kGroupedReadBytes4096 = uint64_t(256) << 20;
+constexpr uint64_t kGroupedReadBytesShared4096 = uint64_t(216) << 20;
+constexpr uint64_t kGroupedReadBytesDear4096 = uint64_t(176) << 20;
 // Whether the layer entry points run a batch of n_tokens on the grouped path.
-bool grouped_preferred(int32_t format, uint64_t n_tokens, uint64_t k, uint64_t hidden, uint64_t inter, uint64_t out_dim);
+bool grouped_preferred(int32_t format, uint64_t n_tokens, uint64_t k, bool shared, uint64_t hidden, uint64_t inter,
+                       uint64_t out_dim);
 // Whether launch_moe_grouped takes this shape.
 bool grouped_supported(int32_t format, uint64_t n_table, uint64_t n_tokens, uint64_t k, uint64_t hidden,
                        uint64_t inter, uint64_t out_dim);

@@ -9,7 +9,7 @@ cover several MFMA column sets."""
 import numpy as np
 import pytest
 
-from objeta_amd import HipError, MoeExecutor
+from objeta_amd import ExpertTable, HipError, MoeExecutor
 from oracle import oracle as orc
 from test_gpu_moe import FP4, IQ3, Q4, Q5, assert_moe_close, device_table, make_experts, oracle_experts
 
@@ -289,3 +289,52 @@ def test_grouped_sets_of_eight(backend, fmt, E, K, T, H, I, O):
 ])
 def test_layer_sets_of_eight_with_shared_expert(backend, fmt, E, K, T, H, I):
     test_layer_batch_runs_grouped_with_shared_expert(backend, fmt, E, K, T, H, I, 0.0)
+
+
+@pytest.mark.parametrize("fmt,K,T,H,I,shared,grouped", [
+    (Q4, 8, 4, 4096, 768, False, False),   # 162 MiB of assigned experts
+    (Q4, 8, 7, 4096, 768, False, True),    # 284
+    (Q4, 8, 8, 2048, 768, False, False),   # 162
+    (Q4, 8, 9, 2048, 768, False, True),    # 182
+    (Q4, 8, 8, 2048, 768, True, True),     # 162 and a shared expert
+    (FP4, 8, 5, 4096, 768, True, False),   # 215 with the shared expert's
+    (FP4, 4, 7, 4096, 1024, True, True),   # 223 with it
+    (Q4, 8, 8, 8192, 384, False, False),   # 324
+    (FP4, 4, 6, 4096, 1024, False, False),  # 153
+    (IQ3, 8, 4, 4096, 1024, False, False),  # 168
+    (IQ3, 6, 6, 4096, 1024, False, True),  # 189
+    (Q5, 8, 4, 2048, 1024, False, True),   # 132
+    (Q4, 4, 7, 2560, 1024, False, False),  # 118
+    (Q4, 4, 8, 2560, 1024, False, True),   # 135
+    (FP4, 4, 4, 3072, 1408, False, False),  # 105
+    (FP4, 4, 5, 3072, 1408, False, True),  # 132
+])
+def test_layer_route_by_assigned_bytes(backend, fmt, K, T, H, I, shared, grouped):
+    """Below 12 tokens and 8 MiB an expert, the layer takes the path that the bytes of its
+    assignments' experts call for: its output is that path's bit for bit, and within the
+    oracle's bar."""
+    E = 12
+    one = make_experts(fmt, 1, H, I, H, seed=3 + fmt, gen="gauss")
+    _, keep = device_table(backend, fmt, one)
+    table = ExpertTable(backend, [tuple(keep)] * E)  # one expert's matrices under every id
+    sh = ExpertTable(backend, [tuple(keep)]) if shared else None
+    w_r = orc.gauss(E * H, 5, 0.02)
+    xs = orc.gauss(T * H, 6, 1.0).reshape(T, H)
+    d_x, d_wr = backend.to_device(xs.ravel()), backend.to_device(w_r)
+    d_out, d_sel, d_grp = (backend.alloc(4 * T * H) for _ in range(3))
+    d_ids, d_w = backend.alloc(4 * T * K), backend.alloc(4 * T * K)
+    moe = MoeExecutor(backend)
+    moe.layer_device(fmt, table, d_wr, None, K, T, d_x, d_x, d_out, d_ids, d_w, H, I, H, shared=sh)
+    moe.selected_device(fmt, table, d_ids, d_w, T, K, d_x, d_x, d_sel, H, I, H, shared=sh)
+    if not shared:
+        moe.grouped_device(fmt, table, d_ids, d_w, T, K, d_x, d_x, d_grp, H, I, H)
+    backend.synchronize()
+    out, sel = d_out.download(np.float32, T * H), d_sel.download(np.float32, T * H)
+    assert np.array_equal(out, sel) != grouped
+    if not shared:
+        assert np.array_equal(out, d_grp.download(np.float32, T * H)) == grouped
+    oe = oracle_experts(fmt, one)
+    rid, rw, _, _ = orc.router(w_r, xs[T - 1], E, H, K, renormalize=True)
+    ref = orc.selected_moe(fmt, oe * E, [(int(i), float(v)) for i, v in zip(rid, rw)], xs[T - 1], H, I, H,
+                           shared=oe[0] if shared else None)
+    assert_moe_close(out.reshape(T, H)[T - 1] - xs[T - 1], ref)
