@@ -70,11 +70,12 @@ struct GroupWs {
 
 // ------------------------------------------------------------------ grouping
 // The shared expert (when given) follows as one more group: member t is token t, its act
-// row n_assign + t.
+// row n_assign + t. Its member sets go after the routed ones in w, or, when wsh.hdr is set
+// (a shared expert of another format, multiplied by a launch of its own), into wsh.
 __device__ void group_assignments(const uint32_t* __restrict__ ids, uint32_t n_assign, uint32_t n_table,
                                   const objeta_hip_expert_ptrs* __restrict__ table,
                                   const objeta_hip_expert_ptrs* __restrict__ shared, uint32_t n_tokens, GroupWs w,
-                                  uint32_t* __restrict__ err) {
+                                  GroupWs wsh, uint32_t* __restrict__ err) {
     __shared__ uint32_t cnt[kGMaxTable];
     __shared__ uint32_t pos[kGMaxTable];
     __shared__ uint32_t sid[kGMaxAssign];
@@ -141,9 +142,14 @@ __device__ void group_assignments(const uint32_t* __restrict__ ids, uint32_t n_a
         }
     }
     const uint32_t n_sh = shared ? (n_tokens + 7) / 8 : 0;
+    const bool apart = wsh.hdr != nullptr;
     if (tid == 0) {
-        w.hdr[0] = tg + (shared ? 1 : 0);
-        w.hdr[1] = ts + n_sh;
+        w.hdr[0] = tg + (shared && !apart ? 1 : 0);
+        w.hdr[1] = ts + (apart ? 0 : n_sh);
+        if (apart) {
+            wsh.hdr[0] = shared ? 1 : 0;
+            wsh.hdr[1] = n_sh;
+        }
     }
     __syncthreads();
     // stable order inside a group: rank among the earlier assignments of the expert
@@ -180,7 +186,7 @@ __device__ void group_assignments(const uint32_t* __restrict__ ids, uint32_t n_a
         mem.y = row(2) | (row(3) << 16);
         mem.z = row(4) | (row(5) << 16);
         mem.w = row(6) | (row(7) << 16);
-        SetRec* dst = &w.sets[si];
+        SetRec* dst = si >= ts && apart ? &wsh.sets[si - ts] : &w.sets[si];
         dst->p = *src;
         *reinterpret_cast<uint4*>(dst->mem) = mem;
     }
@@ -191,12 +197,12 @@ __global__ __launch_bounds__(256) void moe_prepare_kernel(const uint32_t* __rest
                                                           uint32_t n_table,
                                                           const objeta_hip_expert_ptrs* __restrict__ table,
                                                           const objeta_hip_expert_ptrs* __restrict__ shared,
-                                                          uint32_t n_tokens, GroupWs w,
+                                                          uint32_t n_tokens, GroupWs w, GroupWs wsh,
                                                           uint32_t* __restrict__ err, const float* __restrict__ x,
                                                           uint32_t cols, _Float16* __restrict__ xh,
                                                           _Float16* __restrict__ xl, float* __restrict__ xmult,
                                                           uint32_t perm) {
-    if (blockIdx.x == 0) group_assignments(ids, n_assign, n_table, table, shared, n_tokens, w, err);
+    if (blockIdx.x == 0) group_assignments(ids, n_assign, n_table, table, shared, n_tokens, w, wsh, err);
     else split_row(x, cols, xh, xl, xmult, blockIdx.x - 1, perm);
 }
 
@@ -312,19 +318,20 @@ template <class R, int M, uint32_t CH>
 struct Staged {
     static constexpr uint32_t kSeg = Tile<R>::wdw(CH);
     u32x4 w[M][SlabUnits<kSeg>::kN];
-    uint32_t s[M];  // FP4 scales: CH / 128 <= 16 dwords per row
+    uint32_t s[M];   // FP4 scales: CH / 128 <= 16 dwords per row
+    uint32_t ts[M];  // FP8 tile scales of the chunk
 };
 
 // grid = (ceil(rows / 16), gy), 256 threads; workgroup (x, y) takes member sets y,
 // y + gy, ... (the number of sets is known only on the device). GATEUP: rows = inter
-// over the split x rows (cols = hidden), writes act; else rows = out_dim over the split act rows (cols = inter),
-// writes part. Dynamic LDS: two chunk buffers of every matrix.
+// over the split x rows (cols = hidden), writes act (the official SwiGLU when `official` is
+// set); else rows = out_dim over the split act rows (cols = inter), writes part. Dynamic LDS: two chunk buffers of every matrix.
 template <class R, bool GATEUP, bool FULL>
 __global__ __launch_bounds__(256) void moe_grouped_kernel(GroupWs gw, const _Float16* __restrict__ vh,
                                                           const _Float16* __restrict__ vl,
                                                           const float* __restrict__ vmult, float* __restrict__ out,
                                                           uint32_t cols, uint32_t rows, uint32_t k, uint32_t n_assign,
-                                                          float limit) {
+                                                          float limit, uint32_t official) {
     extern __shared__ uint32_t tl[];
     // the cross-wave partial sums reuse the chunk buffers once a set's products are done
     auto red = reinterpret_cast<f32x4 (*)[3][64]>(tl);
@@ -374,8 +381,10 @@ __global__ __launch_bounds__(256) void moe_grouped_kernel(GroupWs gw, const _Flo
                                  Tile<R>::wdw(kc), st.w[t]);
                 if constexpr (Tile<R>::kScales)
                     scale_load(Tile<R>::srow(mt[t], kc0), spitch, r0, rows, Tile<R>::sdw(kc), st.s[t]);
+                if constexpr (Tile<R>::kTileScale) st.ts[t] = Tile<R>::tile_scales(mt[t], r0, kc0, kc);
             }
         };
+        uint32_t ts_cur[kMats] = {};  // the tile scales of the chunk being multiplied
         auto operands = [&](uint32_t kc0, half8 (&xr)[kB]) {
             const uint32_t kc = FULL ? kChunk : (cols - kc0 < kChunk ? cols - kc0 : kChunk);
             const uint32_t nb = kc / 32, per = (nb + 3) / 4;
@@ -395,6 +404,8 @@ __global__ __launch_bounds__(256) void moe_grouped_kernel(GroupWs gw, const _Flo
                 slab_store4<kSeg, FULL>(base, Tile<R>::wdw(kc), st.w[t]);
                 if constexpr (Tile<R>::kScales)
                     scale_store(base + kSlab * kWStride, kSStride, Tile<R>::sdw(kc), st.s[t]);
+                // read only after the products of the previous chunk
+                if constexpr (Tile<R>::kTileScale) ts_cur[t] = st.ts[t];
             }
         };
         f32x4 acc[kMats];
@@ -423,7 +434,7 @@ __global__ __launch_bounds__(256) void moe_grouped_kernel(GroupWs gw, const _Flo
                 for (int i = 0; i < kB; ++i) {
                     if (b0 + static_cast<uint32_t>(i) >= b1) break;
                     float sc;
-                    const half8 bw = Tile<R>::get(wl, sl, 0u, b0 + static_cast<uint32_t>(i), kg, sc);
+                    const half8 bw = Tile<R>::get(wl, sl, ts_cur[t], b0 + static_cast<uint32_t>(i), kg, sc);
                     const f32x4 z = {0.f, 0.f, 0.f, 0.f};
                     const f32x4 r = __builtin_amdgcn_mfma_f32_16x16x32_f16(xa[i], bw, z, 0, 0, 0);
 #pragma unroll
@@ -460,7 +471,7 @@ __global__ __launch_bounds__(256) void moe_grouped_kernel(GroupWs gw, const _Flo
                 const float v0 = (acc[0][2 * q] + acc[0][2 * q + 1]) * mul;
                 if constexpr (GATEUP) {
                     const float v1 = (acc[kMats - 1][2 * q] + acc[kMats - 1][2 * q + 1]) * mul;
-                    if (live) out[static_cast<size_t>(a) * rows + row] = silu_mul(v0, v1, limit);
+                    if (live) out[static_cast<size_t>(a) * rows + row] = swiglu(v0, v1, limit, official);
                 } else {
                     if (live) out[static_cast<size_t>(a) * rows + row] = v0;
                 }
@@ -734,16 +745,16 @@ uint32_t grouped_gy(uint32_t rows, uint32_t max_sets, uint32_t cus) {
 template <class R, bool GATEUP>
 void launch_grouped_products(hipStream_t s, GroupWs gw, const _Float16* vh, const _Float16* vl, const float* vmult,
                              float* dst, uint32_t cols, uint32_t rows, uint32_t k, uint32_t n_assign, float limit,
-                             uint32_t max_sets, uint32_t cus) {
+                             bool official, uint32_t max_sets, uint32_t cus) {
     const size_t lds = (GATEUP ? 2 : 1) * 2 * 4 *
                        static_cast<size_t>(Tile<R>::lds_dw(GATEUP ? Tile<R>::kChunkGU : Tile<R>::kChunkDn));
     const dim3 grid((rows + kSlab - 1) / kSlab, grouped_gy(rows, max_sets, cus));
     if (cols % (GATEUP ? Tile<R>::kChunkGU : Tile<R>::kChunkDn) == 0)
         hipLaunchKernelGGL((moe_grouped_kernel<R, GATEUP, true>), grid, dim3(256), lds, s, gw, vh, vl, vmult, dst, cols,
-                           rows, k, n_assign, limit);
+                           rows, k, n_assign, limit, official ? 1u : 0u);
     else
         hipLaunchKernelGGL((moe_grouped_kernel<R, GATEUP, false>), grid, dim3(256), lds, s, gw, vh, vl, vmult, dst, cols,
-                           rows, k, n_assign, limit);
+                           rows, k, n_assign, limit, official ? 1u : 0u);
 }
 
 template <class R>
@@ -751,12 +762,12 @@ hipError_t launch_grouped(hipStream_t s, GroupWs gw, const _Float16* xh, const _
                           float* act, _Float16* ah, _Float16* al, float* amult, float* part, uint32_t n_assign,
                           uint32_t n_rows, uint32_t max_sets, uint32_t k,
                           uint32_t hidden, uint32_t inter, uint32_t out_dim, float limit, uint32_t cus) {
-    launch_grouped_products<R, true>(s, gw, xh, xl, xmult, act, hidden, inter, k, n_assign, limit, max_sets,
-                                     cus);
+    launch_grouped_products<R, true>(s, gw, xh, xl, xmult, act, hidden, inter, k, n_assign, limit, false,
+                                     max_sets, cus);
     hipLaunchKernelGGL(moe_split_kernel, dim3(n_rows), dim3(256), 0, s, act, inter, ah, al, amult,
                        Tile<R>::kPermuted ? 1u : 0u);
-    launch_grouped_products<R, false>(s, gw, ah, al, amult, part, inter, out_dim, k, n_assign, 0.0f, max_sets,
-                                      cus);
+    launch_grouped_products<R, false>(s, gw, ah, al, amult, part, inter, out_dim, k, n_assign, 0.0f, false,
+                                      max_sets, cus);
     return hipGetLastError();
 }
 
@@ -980,7 +991,7 @@ int32_t launch_moe_grouped(objeta_hip_context* ctx, int32_t format, hipStream_t 
     // the split order follows the weights' order (element order for FP4)
     const bool perm = format == OBJETA_HIP_FP4_E2M1 ? Tile<Fp4Rows>::kPermuted : Tile<QRows<kQ4>>::kPermuted;
     hipLaunchKernelGGL(moe_prepare_kernel, dim3(1 + T), dim3(256), 0, s, ids, A, static_cast<uint32_t>(n_table), table,
-                       shared, T, gw, err, x, H, xh, xl, xmult, perm ? 1u : 0u);
+                       shared, T, gw, GroupWs{nullptr, nullptr}, err, x, H, xh, xl, xmult, perm ? 1u : 0u);
     hipError_t e;
     const uint32_t kk = static_cast<uint32_t>(k);
     switch (format) {
@@ -1007,6 +1018,76 @@ int32_t launch_moe_grouped(objeta_hip_context* ctx, int32_t format, hipStream_t 
         e = hipGetLastError();
     }
     if (e != hipSuccess) OBJ_FAIL(kDriver, action, hipGetErrorString(e));
+    return 0;
+}
+
+// Few assignments on large matrices, as for the plain layer, but the line is set by the FP8
+// shared expert: its rows are the longest, and on the wide products its one set walks them in
+// inter / 32 workgroups. us, wide / here, with the shared expert, below | past the line: 7168 x
+// 2048 top-1, 4 tokens 115 / 92, 14, 117 / 113, top-2, 6, 118 / 113 | 8, 117 / 122, top-4, 3,
+// 122 / 124; 4608 x 1664 top-1, 8, 87 / 79 | top-2, 10, 93 / 97; 4096 x 1408 top-1, 6, 72 / 66 |
+// 20, 73 / 78; 7168 x 768 top-1, 8 | 86 / 88; 2048 x 2048 top-2, 6 | 53 / 55.
+bool official_few(uint64_t n_table, uint64_t n_tokens, uint64_t k, uint64_t hidden, uint64_t inter, uint64_t out_dim) {
+    if (k == 0 || k > 2 || n_table == 0 || n_table > kGMaxTable || n_tokens > 14) return false;
+    if (hidden > (1u << 20) || inter > (1u << 20) || out_dim > (1u << 20)) return false;
+    return n_tokens * k <= 14 && inter > 1024 && hidden * inter >= (uint64_t(5) << 20);
+}
+
+// The official layer (launch_moe_official_grouped) on the sets of eight: the FP8 shared
+// expert's sets apart, in a launch of their own per phase.
+int32_t launch_moe_official_sets(objeta_hip_context* ctx, hipStream_t s, const objeta_hip_expert_ptrs* table,
+                                 uint64_t n_table, const objeta_hip_expert_ptrs* shared, const uint32_t* ids,
+                                 const float* wts, uint64_t n_tokens, uint64_t k, const float* x, float* out,
+                                 uint64_t hidden, uint64_t inter, uint64_t out_dim, float limit,
+                                 uint8_t* inter_values, uint8_t* inter_scales) {
+    const char* action = "launch official FP4 MoE (sets of eight)";
+    const uint32_t T = static_cast<uint32_t>(n_tokens), A = static_cast<uint32_t>(n_tokens * k);
+    const uint32_t NR = A + (shared ? T : 0);       // act rows: routed, then shared
+    const uint32_t NSS = shared ? (T + 7) / 8 : 0;  // shared member sets
+    const uint32_t H = static_cast<uint32_t>(hidden), I = static_cast<uint32_t>(inter), O = static_cast<uint32_t>(out_dim);
+    size_t off = 0;
+    const size_t o_hdr = off; off += align256(16);
+    const size_t o_set = off; off += align256(sizeof(SetRec) * A);
+    const size_t o_hdr2 = off; off += align256(16);
+    const size_t o_set2 = off; off += align256(sizeof(SetRec) * (NSS ? NSS : 1));
+    const size_t o_xd = off; off += align256(4ull * T * H);
+    const size_t o_xm = off; off += align256(4ull * T);
+    const size_t o_am = off; off += align256(4ull * NR);
+    const size_t o_xh = off; off += align256(2ull * T * H);
+    const size_t o_xl = off; off += align256(2ull * T * H);
+    const size_t o_act = off; off += align256(4ull * NR * I);
+    const size_t o_ah = off; off += align256(2ull * NR * I);
+    const size_t o_al = off; off += align256(2ull * NR * I);
+    const size_t o_part = off; off += align256(4ull * NR * O);
+    void* wsp = nullptr;
+    OBJ_TRY(ensure_workspace(ctx, s, kWsGrouped, off, &wsp));
+    char* b = static_cast<char*>(wsp);
+    const GroupWs gw{reinterpret_cast<uint32_t*>(b + o_hdr), reinterpret_cast<SetRec*>(b + o_set)};
+    const GroupWs gws{reinterpret_cast<uint32_t*>(b + o_hdr2), reinterpret_cast<SetRec*>(b + o_set2)};
+    float* xd = reinterpret_cast<float*>(b + o_xd);
+    float* xmult = reinterpret_cast<float*>(b + o_xm);
+    float* amult = reinterpret_cast<float*>(b + o_am);
+    auto* xh = reinterpret_cast<_Float16*>(b + o_xh);
+    auto* xl = reinterpret_cast<_Float16*>(b + o_xl);
+    float* act = reinterpret_cast<float*>(b + o_act);
+    auto* ah = reinterpret_cast<_Float16*>(b + o_ah);
+    auto* al = reinterpret_cast<_Float16*>(b + o_al);
+    float* part = reinterpret_cast<float*>(b + o_part);
+    const uint32_t cus = ctx->info.compute_units > 0 ? static_cast<uint32_t>(ctx->info.compute_units) : 256u;
+    const uint32_t kk = static_cast<uint32_t>(k), perm = Tile<Fp4Rows>::kPermuted ? 1u : 0u;
+    OBJ_TRY(launch_act_quant(s, x, T, H, nullptr, nullptr, xd));
+    hipLaunchKernelGGL(moe_prepare_kernel, dim3(1 + T), dim3(256), 0, s, ids, A, static_cast<uint32_t>(n_table), table,
+                       shared, T, gw, shared ? gws : GroupWs{nullptr, nullptr}, ctx->err_word, xd, H, xh, xl, xmult, perm);
+    launch_grouped_products<Fp4Rows, true>(s, gw, xh, xl, xmult, act, H, I, kk, A, limit, true, A, cus);
+    if (shared) launch_grouped_products<Fp8Rows, true>(s, gws, xh, xl, xmult, act, H, I, kk, A, limit, true, NSS, cus);
+    OBJ_HIP(hipGetLastError(), action);
+    OBJ_TRY(launch_act_quant(s, act, NR, I, inter_values, inter_scales, act));
+    hipLaunchKernelGGL(moe_split_kernel, dim3(NR), dim3(256), 0, s, act, I, ah, al, amult, perm);
+    launch_grouped_products<Fp4Rows, false>(s, gw, ah, al, amult, part, I, O, kk, A, 0.0f, false, A, cus);
+    if (shared) launch_grouped_products<Fp8Rows, false>(s, gws, ah, al, amult, part, I, O, kk, A, 0.0f, false, NSS, cus);
+    launch_moe_combine(s, ids, wts, part, shared ? part + static_cast<size_t>(A) * O : nullptr, nullptr, out, T, kk, O,
+                       static_cast<uint32_t>(n_table));
+    OBJ_HIP(hipGetLastError(), action);
     return 0;
 }
 

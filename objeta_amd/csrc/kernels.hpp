@@ -85,14 +85,23 @@ int32_t launch_moe_official_fp4(objeta_hip_context* ctx, hipStream_t s, const ob
                                 uint8_t* inter_values, uint8_t* inter_scales, const OfficialMarks* marks);
 
 // The same layer on the grouped-token products (wide.hip), for batches of at
-// least kOfficialGroupedMinTokens tokens, or 2 where the per-token kernels would read
-// kOfficialGroupedReadBytes, in the grouped path's limits (us, per-token / grouped: hidden
-// 7168, intermediate 2048, top-8 at 2 tokens, 462 MB, 170 / 151, at 4 318 / 187; hidden
-// 2048, intermediate 768, top-4 at 4 tokens, 59 MB, 30 / 41).
+// least kOfficialGroupedMinTokens tokens, or 3 (2) where the per-token kernels would read
+// kOfficialGroupedReadBytes (kOfficialGroupedReadBytes2: two tokens share few experts), in
+// the grouped path's limits. us, per-token / grouped: hidden 7168, intermediate 2048 at 2
+// tokens, top-4, 262 MiB, 106 / 117, top-8, 441 MiB, 172 / 151, at 4 317 / 167; 4608 x 1664
+// top-4 at 4 tokens, 274 MiB, 128 / 91; 2048 x 768 top-8 at 5 tokens, 118 MiB, 41 / 45.
 constexpr uint64_t kOfficialGroupedMinTokens = 6;
 constexpr uint64_t kOfficialGroupedReadBytes = uint64_t(256) << 20;
+constexpr uint64_t kOfficialGroupedReadBytes2 = uint64_t(288) << 20;
 bool official_grouped_supported(uint64_t n_table, uint64_t n_tokens, uint64_t k, uint64_t hidden, uint64_t inter,
                                 uint64_t out_dim);
+// Whether launch_moe_official_grouped runs the batch on the sets of eight of grouped.hip.
+bool official_few(uint64_t n_table, uint64_t n_tokens, uint64_t k, uint64_t hidden, uint64_t inter, uint64_t out_dim);
+int32_t launch_moe_official_sets(objeta_hip_context* ctx, hipStream_t s, const objeta_hip_expert_ptrs* table,
+                                 uint64_t n_table, const objeta_hip_expert_ptrs* shared, const uint32_t* ids,
+                                 const float* wts, uint64_t n_tokens, uint64_t k, const float* x, float* out,
+                                 uint64_t hidden, uint64_t inter, uint64_t out_dim, float limit,
+                                 uint8_t* inter_values, uint8_t* inter_scales);
 int32_t launch_moe_official_grouped(objeta_hip_context* ctx, hipStream_t s, const objeta_hip_expert_ptrs* table,
                                     uint64_t n_table, const objeta_hip_expert_ptrs* shared, const uint32_t* ids,
                                     const float* wts, uint64_t n_tokens, uint64_t k, const float* x, float* out,

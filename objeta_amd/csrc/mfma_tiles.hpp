@@ -220,8 +220,10 @@ struct Tile<Fp8Rows> {
     static constexpr bool kPermuted = false;
     static constexpr bool kScales = false;
     static constexpr bool kTileScale = true;
+    static constexpr uint32_t kChunkGU = 256, kChunkDn = 256;
     static constexpr __host__ __device__ uint32_t wdw(uint32_t kc) { return kc / 4; }  // kc bytes
     static constexpr __host__ __device__ uint32_t sdw(uint32_t) { return 0; }
+    static constexpr __host__ __device__ uint32_t lds_dw(uint32_t kc) { return kSlab * (wdw(kc) + 4); }
     static __device__ __forceinline__ size_t wpitch(const Fp8Rows& m) { return m.wrow; }
     static __device__ __forceinline__ size_t spitch(const Fp8Rows&) { return 0; }
     static __device__ __forceinline__ const uint8_t* wrow(const Fp8Rows& m, uint32_t c0) { return m.w + c0; }

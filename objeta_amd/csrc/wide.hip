@@ -800,7 +800,8 @@ bool official_grouped_supported(uint64_t n_table, uint64_t n_tokens, uint64_t k,
     if (n_tokens < 2 || !wide_shape(OBJETA_HIP_FP4_E2M1, n_table, k, hidden, inter, out_dim)) return false;
     const uint64_t matrices = 2 * inter * hidden + out_dim * inter;  // an expert's weights
     if (n_tokens < kOfficialGroupedMinTokens &&
-        n_tokens * (k * (matrices / 32 * 17) + matrices) < kOfficialGroupedReadBytes)
+        n_tokens * (k * (matrices / 32 * 17) + matrices) <
+            (n_tokens == 2 ? kOfficialGroupedReadBytes2 : kOfficialGroupedReadBytes))
         return false;
     return matrices_fit(OBJETA_HIP_FP4_E2M1, true, hidden, inter, out_dim) && n_tokens <= launch_tokens(k, hidden, inter);
 }
@@ -823,6 +824,9 @@ int32_t launch_moe_official_grouped(objeta_hip_context* ctx, hipStream_t s, cons
     static_assert(Tile<Fp4Rows>::kPermuted == Tile<Fp8Rows>::kPermuted, "one activation order for both tiles");
     if (!official_grouped_supported(n_table, n_tokens, k, hidden, inter, out_dim))
         OBJ_FAIL(kUnsupported, action, "shape outside the grouped official path");
+    if (official_few(n_table, n_tokens, k, hidden, inter, out_dim))
+        return launch_moe_official_sets(ctx, s, table, n_table, shared, ids, wts, n_tokens, k, x, out, hidden, inter,
+                                        out_dim, limit, inter_values, inter_scales);
     const uint32_t T = static_cast<uint32_t>(n_tokens), A = static_cast<uint32_t>(n_tokens * k);
     const uint32_t NR = A + (shared ? T : 0);  // act rows: routed, then shared
     const uint32_t M = WorkOfficial::kMembers;

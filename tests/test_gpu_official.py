@@ -344,6 +344,26 @@ def test_official_layer_batch_grouped(backend, T, k, with_shared):
     check_official(out, q, s, experts, shared, selections, xs, hidden, inter, out_dim)
 
 
+@pytest.mark.parametrize("T,k,hidden,inter,with_shared", [
+    (6, 2, 4736, 1152, True),    # two tokens' sets; every chunk width leaves a short chunk
+    (14, 1, 4736, 1152, False),
+    (14, 1, 4096, 1536, True),   # whole chunks; the shared expert in two sets, the second of six
+    (6, 4, 7168, 1408, True),    # past the few: the wide products' 128-row work with a short chunk
+])
+def test_official_layer_few_assignments_on_large_matrices(backend, T, k, hidden, inter, with_shared):
+    """At most 14 assignments of top-1 or top-2 on large matrices: sets of eight, the FP8
+    shared expert's in launches of their own; more run on the wide products."""
+    out_dim, n = hidden, 5
+    experts = [fp4_random_expert(hidden, inter, out_dim, 500 + 3 * e) for e in range(n)]
+    shared = fp8_random_expert(hidden, inter, out_dim, 78) if with_shared else None
+    rng = np.random.default_rng(T * 7 + k)
+    selections = [[(int(e), float(w)) for e, w in zip(rng.choice(n, k, replace=False),
+                                                      rng.dirichlet(np.ones(k)).astype(F32))] for _ in range(T)]
+    xs = orc.gauss(T * hidden, 92 + T, 2.0).reshape(T, hidden)
+    out, q, s = run_official(backend, experts, shared, selections, xs, hidden, inter, out_dim)
+    check_official(out, q, s, experts, shared, selections, xs, hidden, inter, out_dim)
+
+
 def test_official_layer_batch_repeats_limits_and_bad_id(backend):
     """The grouped official path with a token that selects one expert twice, the
     clamp at 0.5 and at 0, and an out-of-table id (error bit 1, that token's output
