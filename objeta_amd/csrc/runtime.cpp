@@ -99,9 +99,17 @@ int32_t ensure_workspace(objeta_hip_context* ctx, hipStream_t stream, int slot, 
     }
     OBJ_TRY(fail_if_capturing(stream, "grow workspace",
                               strf("workspace of %zu bytes (have %zu)", bytes, ws.bytes)));
+    // by half again at least, so that sizes climbing call by call leave regions of at most
+    // twice the last one's bytes retired
     size_t grow = bytes < (size_t(1) << 20) ? (size_t(1) << 20) : bytes;
+    if (grow < ws.bytes + ws.bytes / 2) grow = ws.bytes + ws.bytes / 2;
     void* p = nullptr;
-    OBJ_HIP(hipMalloc(&p, grow), "allocate workspace");
+    if (grow > bytes && hipMalloc(&p, grow) != hipSuccess) {
+        (void)hipGetLastError();
+        p = nullptr;
+        grow = bytes;
+    }
+    if (!p) OBJ_HIP(hipMalloc(&p, grow), "allocate workspace");
     // epoch-tagged words in a workspace must start at zero
     OBJ_HIP(hipMemsetAsync(p, 0, grow, stream), "clear workspace");
     OBJ_HIP(hipStreamSynchronize(stream), "clear workspace");

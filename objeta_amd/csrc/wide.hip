@@ -879,50 +879,69 @@ int32_t launch_moe_official_grouped(objeta_hip_context* ctx, hipStream_t s, cons
 }
 
 bool gemv_wide_supported(int32_t format, uint64_t rows, uint64_t cols, uint64_t batch) {
-    return batch >= kGemvWideMinBatch && below_2g(rows, cols) && below_2g(batch, 2 * cols) && (batch + 15) / 16 <= 65535;
+    return batch >= kGemvWideMinBatch && batch <= 0x7FFFFFFFull && below_2g(rows, cols);
 }
 
 namespace {
+
+// Vectors per launch of the batched GEMV: equal multiples of 32 whose two split parts take
+// at most 256 MiB (64 vectors at 2^20 columns), so the workspace is bounded however many
+// vectors a call brings: 16384 vectors of 4096 columns go in one. (With 64 MiB, 1200 vectors
+// of 14336 columns by 4096 rows took 617 us in two launches, 506 in one.)
+uint32_t gemv_slice(uint32_t batch, uint32_t cols) {
+    const uint32_t most = (64u << 20) / cols / 32 * 32;
+    if (batch <= most) return batch;
+    const uint32_t n = (batch + most - 1) / most;
+    return ((batch + n - 1) / n + 31) / 32 * 32;
+}
 
 template <class R, class K>
 int32_t launch_gemv_wide_t(objeta_hip_context* ctx, hipStream_t s, const void* w, const void* ws, const float* x, float* y,
                            uint32_t rows, uint32_t cols, uint32_t batch) {
     const uint32_t cus = ctx->info.compute_units > 0 ? static_cast<uint32_t>(ctx->info.compute_units) : 256u;
-    const uint32_t nrb = row_blocks<K, kWGemv>(rows), ng = (batch + K::kMembers - 1) / K::kMembers;
-    // column ranges for about two workgroups per CU, of at least 512 columns (in units of
-    // the larger chunk)
-    const uint32_t units = (cols + 255) / 256;
-    uint32_t ks = (2 * cus + nrb * ng - 1) / (nrb * ng);
-    if (ks > (units + 1) / 2) ks = (units + 1) / 2;
-    WideArgs g{};
-    g.range = 256 * ((units + ks - 1) / ks);
-    ks = (cols + g.range - 1) / g.range;
+    const uint32_t nrb = row_blocks<K, kWGemv>(rows);
+    const uint32_t slice = gemv_slice(batch, cols);
+    // at most half as many column ranges as the columns have units of 256
+    const uint32_t units = (cols + 255) / 256, ks_max = (units + 1) / 2;
     size_t off = 0;
-    const size_t o_xm = off; off += al256(4ull * batch);
-    const size_t o_xh = off; off += al256(2ull * batch * cols);
-    const size_t o_xl = off; off += al256(2ull * batch * cols);
-    const size_t o_part = off; off += ks > 1 ? al256(4ull * ks * batch * rows) : 0;
+    const size_t o_xm = off; off += al256(4ull * slice);
+    const size_t o_xh = off; off += al256(2ull * slice * cols);
+    const size_t o_xl = off; off += al256(2ull * slice * cols);
+    // partial sums: several ranges only while row blocks x vector groups are below 2 cus, so
+    // below 4 cus workgroups in all (a bound that does not fall as the batch grows)
+    const uint64_t tiles = 4ull * cus * K::kMembers * K::kRows, all = static_cast<uint64_t>(ks_max) * slice * rows;
+    const size_t o_part = off; off += ks_max > 1 ? al256(4 * (tiles < all ? tiles : all)) : 0;
     void* wsp = nullptr;
     OBJ_TRY(ensure_workspace(ctx, s, kWsGemv, off, &wsp));
     char* b = static_cast<char*>(wsp);
     float* xmult = reinterpret_cast<float*>(b + o_xm);
     auto* xh = reinterpret_cast<_Float16*>(b + o_xh);
     auto* xl = reinterpret_cast<_Float16*>(b + o_xl);
+    WideArgs g{};
     g.w0 = w;
     g.s0 = ws;
     g.vh = xh;
     g.vl = xl;
     g.vmult = xmult;
-    g.out = ks > 1 ? reinterpret_cast<float*>(b + o_part) : y;
     g.cols = cols;
     g.rows = rows;
-    g.n_vec = batch;
     g.nrb = nrb;
-    hipLaunchKernelGGL(wide_split_kernel, dim3(batch), dim3(256), 0, s, x, cols, xh, xl, xmult,
-                       Tile<R>::kPermuted ? 1u : 0u);
-    launch_wide_products<R, K, kWGemv>(s, dim3(nrb, ks, ng), g);
-    if (ks > 1) launch_gemv_reduce(s, g.out, y, rows, batch, ks);
-    OBJ_HIP(hipGetLastError(), "launch batched GEMV (wide)");
+    for (uint32_t v0 = 0; v0 < batch; v0 += slice) {
+        const uint32_t n = batch - v0 < slice ? batch - v0 : slice, ng = (n + K::kMembers - 1) / K::kMembers;
+        // column ranges for about two workgroups per CU, of at least 512 columns
+        uint32_t ks = (2 * cus + nrb * ng - 1) / (nrb * ng);
+        if (ks > ks_max) ks = ks_max;
+        g.range = 256 * ((units + ks - 1) / ks);
+        ks = (cols + g.range - 1) / g.range;
+        float* const ys = y + static_cast<size_t>(v0) * rows;
+        g.out = ks > 1 ? reinterpret_cast<float*>(b + o_part) : ys;
+        g.n_vec = n;
+        hipLaunchKernelGGL(wide_split_kernel, dim3(n), dim3(256), 0, s, x + static_cast<size_t>(v0) * cols, cols, xh, xl,
+                           xmult, Tile<R>::kPermuted ? 1u : 0u);
+        launch_wide_products<R, K, kWGemv>(s, dim3(nrb, ks, ng), g);
+        if (ks > 1) launch_gemv_reduce(s, g.out, ys, rows, n, ks);
+        OBJ_HIP(hipGetLastError(), "launch batched GEMV (wide)");
+    }
     return 0;
 }
 

@@ -7,8 +7,9 @@ import ctypes as C
 
 import numpy as np
 import pytest
+import torch
 
-from objeta_amd import MoeExecutor, QGemvShape, QuantBackend, QuantFormat
+from objeta_amd import HipBackend, MoeExecutor, QGemvShape, QuantBackend, QuantFormat
 from objeta_amd.api import check
 from oracle import oracle as orc
 from test_gpu_grouped import skewed_selection
@@ -37,6 +38,27 @@ def test_gemv_wide(backend, fmt, rows, cols, batch):
     for t in range(batch):
         xt = xs[t * cols:(t + 1) * cols]
         _assert_close(y[t], orc.gemv(int(fmt), q, xt, rows, cols), q, xt, fmt, rows, cols)
+
+
+def test_gemv_wide_slices(backend):
+    """2^20 columns: launches of 64 vectors, 70 in two."""
+    test_gemv_wide(backend, QuantFormat.Q4_0, 3, 1 << 20, 70)
+
+
+def test_gemv_workspace_of_climbing_batches():
+    """Batches that climb call by call: the workspace and what it replaced stay within four
+    times the largest call's split vectors (64 MiB here)."""
+    be = HipBackend(0, 1)
+    rows, cols, step, most = 64, 4096, 128, 4096
+    q = be.to_device(orc.quantize_matrix(0, orc.gauss(rows * cols, 3, 0.02), rows, cols))
+    x, y = be.alloc(4 * most * cols), be.alloc(4 * most * rows)
+    quant = QuantBackend(be)
+    free = torch.cuda.mem_get_info()[0]
+    for batch in range(step, most + 1, step):
+        quant.launch_kernel(QuantFormat.Q4_0, None, q, x, y, QGemvShape.new(QuantFormat.Q4_0, rows, cols), batch=batch)
+    be.synchronize()
+    assert free - torch.cuda.mem_get_info()[0] <= 4 * (4 * most * cols)
+    be.close()
 
 
 @pytest.mark.parametrize("fmt,cols", [(QuantFormat.Q4_0, 4096), (QuantFormat.Q5_0, 4160), (QuantFormat.IQ3_0, 4096)])
