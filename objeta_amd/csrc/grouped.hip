@@ -731,8 +731,6 @@ __global__ __launch_bounds__(256) void moe_combine_kernel(const uint32_t* __rest
     out[static_cast<size_t>(t) * out_dim + r] = acc;
 }
 
-size_t align256(size_t v) { return (v + 255) & ~size_t(255); }
-
 // about sixteen workgroups per CU over all slabs, at most one per member set
 uint32_t grouped_gy(uint32_t rows, uint32_t max_sets, uint32_t cus) {
     const uint32_t slabs = (rows + kSlab - 1) / kSlab;
@@ -834,21 +832,27 @@ hipError_t launch_gemv_mfma_t(hipStream_t s, const void* w, const void* ws, cons
 }
 }  // namespace
 
+size_t gemv_passes_bytes(uint64_t rows, uint64_t cols, uint64_t batch) {
+    const uint64_t ks = (cols + kGemvRange - 1) / kGemvRange;
+    return ks > 1 ? 4 * ks * (batch < 8 ? batch : 8) * rows : 0;
+}
+
 int32_t launch_gemv_mfma(objeta_hip_context* ctx, hipStream_t s, int32_t format, const void* w, const void* ws,
                          const float* x, float* y, uint64_t rows, uint64_t cols, uint64_t batch) {
     const char* action = "launch batched GEMV (MFMA)";
     if (!gemv_mfma_supported(format, rows, cols, batch, w, x))
         OBJ_FAIL(kUnsupported, action, "shape, batch or alignment outside the MFMA GEMV");
-    if (gemv_wide_supported(format, rows, cols, batch))
+    // (under capture without its workspace, the passes below, which need less or none)
+    if (gemv_wide_supported(format, rows, cols, batch) &&
+        workspace_ready(ctx, s, kWsGemv, gemv_wide_bytes(ctx, format, rows, cols, batch)))
         return launch_gemv_wide(ctx, s, format, w, ws, x, y, rows, cols, batch);
     const uint32_t R = static_cast<uint32_t>(rows), K = static_cast<uint32_t>(cols);
     const uint32_t ks = (K + kGemvRange - 1) / kGemvRange;  // column ranges
-    const uint32_t nvmax = static_cast<uint32_t>(batch < 8 ? batch : 8);
     const uint32_t cus = ctx->info.compute_units > 0 ? static_cast<uint32_t>(ctx->info.compute_units) : 256u;
     float* part = nullptr;
     if (ks > 1) {
         void* wsp = nullptr;
-        OBJ_TRY(ensure_workspace(ctx, s, kWsGemv, 4ull * ks * nvmax * R, &wsp));
+        OBJ_TRY(ensure_workspace(ctx, s, kWsGemv, gemv_passes_bytes(rows, cols, batch), &wsp));
         part = static_cast<float*>(wsp);
     }
     for (uint64_t done = 0; done < batch; done += 8) {
@@ -910,6 +914,55 @@ bool grouped_supported(int32_t format, uint64_t n_table, uint64_t n_tokens, uint
     return format != OBJETA_HIP_FP4_E2M1;
 }
 
+namespace {
+// The layout for T tokens; the pointers of w are set when base is.
+size_t grouped_layout(uint64_t T, uint64_t k, uint64_t n_table, bool shared, uint64_t H, uint64_t I, uint64_t O,
+                      bool official, char* base, GroupedWs* w) {
+    const uint64_t A = T * k, NR = A + (shared ? T : 0), n8 = shared ? (T + 7) / 8 : 0, n16 = shared ? (T + 15) / 16 : 0;
+    auto larger = [](uint64_t a, uint64_t b) { return a > b ? a : b; };
+    auto whole = [](uint64_t n) { return (n + 7) & ~uint64_t(7); };  // rounds of the eight XCDs
+    size_t off = 0;
+    auto take = [&](size_t bytes) {
+        char* const at = base ? base + off : nullptr;
+        off += (bytes + 255) & ~size_t(255);
+        return at;
+    };
+    GroupedWs g;
+    g.hdr = reinterpret_cast<uint32_t*>(take(16));
+    g.sets = take(larger(sizeof(SetRec) * (A + n8), kWideSetBytes * whole((A < n_table ? A : n_table) + A / 16 + n16)));
+    g.shared_sets = take(larger(sizeof(SetRec) * n8, kWideSetBytes * whole(n16)));
+    g.xd = reinterpret_cast<float*>(take(official ? 4 * T * H : 0));
+    g.xmult = reinterpret_cast<float*>(take(4 * T));
+    g.amult = reinterpret_cast<float*>(take(4 * NR));
+    g.xh = reinterpret_cast<_Float16*>(take(2 * T * H));
+    g.xl = reinterpret_cast<_Float16*>(take(2 * T * H));
+    g.act = reinterpret_cast<float*>(take(4 * NR * I));
+    g.ah = reinterpret_cast<_Float16*>(take(2 * NR * I));
+    g.al = reinterpret_cast<_Float16*>(take(2 * NR * I));
+    g.part = reinterpret_cast<float*>(take(4 * NR * O));
+    if (w) *w = g;
+    return off;
+}
+}  // namespace
+
+int32_t grouped_workspace(objeta_hip_context* ctx, hipStream_t s, uint64_t n_tokens, uint64_t k, uint64_t n_table,
+                          bool shared, uint64_t hidden, uint64_t inter, uint64_t out_dim, bool official, GroupedWs& w) {
+    void* p = nullptr;
+    OBJ_TRY(ensure_workspace(ctx, s, kWsGrouped,
+                             grouped_layout(n_tokens, k, n_table, shared, hidden, inter, out_dim, official, nullptr, nullptr), &p));
+    (void)grouped_layout(n_tokens, k, n_table, shared, hidden, inter, out_dim, official, static_cast<char*>(p), &w);
+    return 0;
+}
+
+bool grouped_ready(objeta_hip_context* ctx, hipStream_t s, int32_t format, uint64_t n_table, uint64_t n_tokens, uint64_t k,
+                   bool shared, uint64_t hidden, uint64_t inter, uint64_t out_dim, bool official) {
+    uint64_t t = n_tokens;
+    if (wide_supported(format, n_table, n_tokens, k, hidden, inter, out_dim) && t > wide_tokens(k, hidden, inter))
+        t = wide_tokens(k, hidden, inter);
+    return workspace_ready(ctx, s, kWsGrouped,
+                           grouped_layout(t, k, n_table, shared, hidden, inter, out_dim, official, nullptr, nullptr));
+}
+
 bool grouped_preferred(int32_t format, uint64_t n_tokens, uint64_t k, bool shared, uint64_t hidden, uint64_t inter,
                        uint64_t out_dim) {
     if (n_tokens >= kGroupedMinTokens) return true;
@@ -962,30 +1015,11 @@ int32_t launch_moe_grouped(objeta_hip_context* ctx, int32_t format, hipStream_t 
     const uint32_t NR = A + (shared ? T : 0);                  // act rows: routed, then shared
     const uint32_t NS = A + (shared ? (T + 7) / 8 : 0);        // member sets at most
     const uint32_t H = static_cast<uint32_t>(hidden), I = static_cast<uint32_t>(inter), O = static_cast<uint32_t>(out_dim);
-    // workspace: set records, split x, act, split act, per-assignment down rows
-    size_t off = 0;
-    const size_t o_hdr = off; off += align256(16);
-    const size_t o_set = off; off += align256(sizeof(SetRec) * NS);
-    const size_t o_xm = off; off += align256(4ull * T);
-    const size_t o_am = off; off += align256(4ull * NR);
-    const size_t o_xh = off; off += align256(2ull * T * H);
-    const size_t o_xl = off; off += align256(2ull * T * H);
-    const size_t o_act = off; off += align256(4ull * NR * I);
-    const size_t o_ah = off; off += align256(2ull * NR * I);
-    const size_t o_all = off; off += align256(2ull * NR * I);
-    const size_t o_part = off; off += align256(4ull * NR * O);
-    void* wsp = nullptr;
-    OBJ_TRY(ensure_workspace(ctx, s, kWsGrouped, off, &wsp));
-    char* b = static_cast<char*>(wsp);
-    GroupWs gw{reinterpret_cast<uint32_t*>(b + o_hdr), reinterpret_cast<SetRec*>(b + o_set)};
-    float* amult = reinterpret_cast<float*>(b + o_am);
-    float* xmult = reinterpret_cast<float*>(b + o_xm);
-    auto* xh = reinterpret_cast<_Float16*>(b + o_xh);
-    auto* xl = reinterpret_cast<_Float16*>(b + o_xl);
-    float* act = reinterpret_cast<float*>(b + o_act);
-    auto* ah = reinterpret_cast<_Float16*>(b + o_ah);
-    auto* al = reinterpret_cast<_Float16*>(b + o_all);
-    float* part = reinterpret_cast<float*>(b + o_part);
+    GroupedWs w;
+    OBJ_TRY(grouped_workspace(ctx, s, T, k, n_table, shared != nullptr, hidden, inter, out_dim, false, w));
+    const GroupWs gw{w.hdr, static_cast<SetRec*>(w.sets)};
+    float *const amult = w.amult, *const xmult = w.xmult, *const act = w.act, *const part = w.part;
+    _Float16 *const xh = w.xh, *const xl = w.xl, *const ah = w.ah, *const al = w.al;
     uint32_t* err = ctx->err_word;
     const uint32_t cus = ctx->info.compute_units > 0 ? static_cast<uint32_t>(ctx->info.compute_units) : 256u;
     // the split order follows the weights' order (element order for FP4)
@@ -1045,34 +1079,11 @@ int32_t launch_moe_official_sets(objeta_hip_context* ctx, hipStream_t s, const o
     const uint32_t NR = A + (shared ? T : 0);       // act rows: routed, then shared
     const uint32_t NSS = shared ? (T + 7) / 8 : 0;  // shared member sets
     const uint32_t H = static_cast<uint32_t>(hidden), I = static_cast<uint32_t>(inter), O = static_cast<uint32_t>(out_dim);
-    size_t off = 0;
-    const size_t o_hdr = off; off += align256(16);
-    const size_t o_set = off; off += align256(sizeof(SetRec) * A);
-    const size_t o_hdr2 = off; off += align256(16);
-    const size_t o_set2 = off; off += align256(sizeof(SetRec) * (NSS ? NSS : 1));
-    const size_t o_xd = off; off += align256(4ull * T * H);
-    const size_t o_xm = off; off += align256(4ull * T);
-    const size_t o_am = off; off += align256(4ull * NR);
-    const size_t o_xh = off; off += align256(2ull * T * H);
-    const size_t o_xl = off; off += align256(2ull * T * H);
-    const size_t o_act = off; off += align256(4ull * NR * I);
-    const size_t o_ah = off; off += align256(2ull * NR * I);
-    const size_t o_al = off; off += align256(2ull * NR * I);
-    const size_t o_part = off; off += align256(4ull * NR * O);
-    void* wsp = nullptr;
-    OBJ_TRY(ensure_workspace(ctx, s, kWsGrouped, off, &wsp));
-    char* b = static_cast<char*>(wsp);
-    const GroupWs gw{reinterpret_cast<uint32_t*>(b + o_hdr), reinterpret_cast<SetRec*>(b + o_set)};
-    const GroupWs gws{reinterpret_cast<uint32_t*>(b + o_hdr2), reinterpret_cast<SetRec*>(b + o_set2)};
-    float* xd = reinterpret_cast<float*>(b + o_xd);
-    float* xmult = reinterpret_cast<float*>(b + o_xm);
-    float* amult = reinterpret_cast<float*>(b + o_am);
-    auto* xh = reinterpret_cast<_Float16*>(b + o_xh);
-    auto* xl = reinterpret_cast<_Float16*>(b + o_xl);
-    float* act = reinterpret_cast<float*>(b + o_act);
-    auto* ah = reinterpret_cast<_Float16*>(b + o_ah);
-    auto* al = reinterpret_cast<_Float16*>(b + o_al);
-    float* part = reinterpret_cast<float*>(b + o_part);
+    GroupedWs w;
+    OBJ_TRY(grouped_workspace(ctx, s, T, k, n_table, shared != nullptr, hidden, inter, out_dim, true, w));
+    const GroupWs gw{w.hdr, static_cast<SetRec*>(w.sets)}, gws{w.hdr + 2, static_cast<SetRec*>(w.shared_sets)};
+    float *const xd = w.xd, *const xmult = w.xmult, *const amult = w.amult, *const act = w.act, *const part = w.part;
+    _Float16 *const xh = w.xh, *const xl = w.xl, *const ah = w.ah, *const al = w.al;
     const uint32_t cus = ctx->info.compute_units > 0 ? static_cast<uint32_t>(ctx->info.compute_units) : 256u;
     const uint32_t kk = static_cast<uint32_t>(k), perm = Tile<Fp4Rows>::kPermuted ? 1u : 0u;
     OBJ_TRY(launch_act_quant(s, x, T, H, nullptr, nullptr, xd));

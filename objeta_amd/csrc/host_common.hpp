@@ -125,6 +125,10 @@ int32_t stream_scratch(objeta_hip_context* ctx, hipStream_t stream, StreamScratc
 // Makes sure workspace region `slot` of `stream` holds at least `bytes` and returns
 // it in *out; fails (Unsupported) if it would have to grow while `stream` is capturing.
 int32_t ensure_workspace(objeta_hip_context* ctx, hipStream_t stream, int slot, size_t bytes, void** out);
+// Whether ensure_workspace would succeed without allocating, or may allocate (no capture).
+bool workspace_ready(objeta_hip_context* ctx, hipStream_t stream, int slot, size_t bytes);
+// ensure_workspace for a region that a later captured call may need; nothing while capturing.
+int32_t offer_workspace(objeta_hip_context* ctx, hipStream_t stream, int slot, size_t bytes);
 // Releases the device memory of every cache still alive on `ctx` (the caches stay
 // valid as accounting-only objects until destroyed).
 void detach_caches(objeta_hip_context* ctx);

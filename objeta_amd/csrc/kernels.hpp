@@ -161,6 +161,23 @@ constexpr uint64_t kGroupedReadBytes2048 = uint64_t(168) << 20;
 constexpr uint64_t kGroupedReadBytes4096 = uint64_t(256) << 20;
 constexpr uint64_t kGroupedReadBytesShared4096 = uint64_t(216) << 20;
 constexpr uint64_t kGroupedReadBytesDear4096 = uint64_t(176) << 20;
+// The workspace of a grouped launch, one layout for every form (sets of eight, wide
+// products, official layer): a call prepares what any smaller batch of the shape needs under
+// capture, whichever form that one takes.
+struct GroupedWs {
+    uint32_t* hdr;             // 4 words
+    void *sets, *shared_sets;  // set records; those of a shared expert apart
+    float *xd, *xmult, *amult, *act, *part;
+    _Float16 *xh, *xl, *ah, *al;
+};
+constexpr size_t kWideSetBytes = 128;  // a set record of the wide products
+int32_t grouped_workspace(objeta_hip_context* ctx, hipStream_t s, uint64_t n_tokens, uint64_t k, uint64_t n_table,
+                          bool shared, uint64_t hidden, uint64_t inter, uint64_t out_dim, bool official, GroupedWs& w);
+// Whether launch_moe_grouped (launch_moe_official_grouped) has its workspace or may make it.
+bool grouped_ready(objeta_hip_context* ctx, hipStream_t s, int32_t format, uint64_t n_table, uint64_t n_tokens, uint64_t k,
+                   bool shared, uint64_t hidden, uint64_t inter, uint64_t out_dim, bool official);
+// Tokens of one launch of the wide products.
+uint64_t wide_tokens(uint64_t k, uint64_t hidden, uint64_t inter);
 // Whether the layer entry points run a batch of n_tokens on the grouped path.
 bool grouped_preferred(int32_t format, uint64_t n_tokens, uint64_t k, bool shared, uint64_t hidden, uint64_t inter,
                        uint64_t out_dim);
@@ -193,6 +210,9 @@ int32_t launch_moe_wide(objeta_hip_context* ctx, int32_t format, hipStream_t s, 
 // 35.4, 128 84 / 275.
 constexpr uint64_t kGemvWideMinBatch = 9;
 bool gemv_wide_supported(int32_t format, uint64_t rows, uint64_t cols, uint64_t batch);
+// Bytes of its workspace, and of launch_gemv_mfma's passes of 8 vectors.
+size_t gemv_passes_bytes(uint64_t rows, uint64_t cols, uint64_t batch);
+size_t gemv_wide_bytes(objeta_hip_context* ctx, int32_t format, uint64_t rows, uint64_t cols, uint64_t batch);
 int32_t launch_gemv_wide(objeta_hip_context* ctx, hipStream_t s, int32_t format, const void* w, const void* ws,
                          const float* x, float* y, uint64_t rows, uint64_t cols, uint64_t batch);
 // out = resid + sum_j w_j part_j (+ shared part), and the sum of a GEMV's column ranges.

@@ -814,13 +814,21 @@ int32_t launch_moe_official_fp4(objeta_hip_context* ctx, hipStream_t s, const ob
     }
     // a batch: every routed expert's matrices (and the shared expert's) read once per
     // member set instead of once per (token, slot)
-    if (official_grouped_supported(n_table, n_tokens, k, hidden, inter, out_dim))
+    auto per_token_bytes = [&](uint64_t tokens) {  // x dequantized, then the intermediates
+        return ((static_cast<size_t>(tokens * hidden) * sizeof(float) + 255) & ~size_t(255)) +
+               static_cast<size_t>(tokens * kk * inter) * sizeof(float) + 64;
+    };
+    if (official_grouped_supported(n_table, n_tokens, k, hidden, inter, out_dim) &&
+        grouped_ready(ctx, s, OBJETA_HIP_FP4_E2M1, n_table, n_tokens, k, shared != nullptr, hidden, inter, out_dim, true)) {
+        // and what the batches below kOfficialGroupedMinTokens need on the per-token kernels
+        OBJ_TRY(offer_workspace(ctx, s, kWsOfficial,
+                                per_token_bytes(n_tokens < kOfficialGroupedMinTokens ? n_tokens : kOfficialGroupedMinTokens - 1)));
         return launch_moe_official_grouped(ctx, s, table, n_table, shared, ids, wts, n_tokens, k, x, out, hidden,
                                            inter, out_dim, limit, inter_values, inter_scales, marks);
+    }
     const size_t xb = (static_cast<size_t>(n_tokens * hidden) * sizeof(float) + 255) & ~size_t(255);
-    const size_t ab = static_cast<size_t>(n_tokens * kk * inter) * sizeof(float);
     void* ws = nullptr;
-    OBJ_TRY(ensure_workspace(ctx, s, kWsOfficial, xb + ab + 64, &ws));
+    OBJ_TRY(ensure_workspace(ctx, s, kWsOfficial, per_token_bytes(n_tokens), &ws));
     float* xd = static_cast<float*>(ws);
     float* act = reinterpret_cast<float*>(static_cast<char*>(ws) + xb);
     float* act_sh = act + n_tokens * k * inter;
@@ -898,10 +906,14 @@ int32_t bind_static_scratch(objeta_hip_context* ctx) {
     return 0;
 }
 
+static size_t act_scratch_bytes(uint64_t n_tokens, uint64_t k, uint64_t inter) {
+    return static_cast<size_t>(n_tokens * k * inter) * sizeof(float) + 64;
+}
+
 int32_t moe_act_scratch(objeta_hip_context* ctx, hipStream_t s, uint64_t n_tokens, uint64_t k, uint64_t inter,
                         float** out) {
     void* p = nullptr;
-    OBJ_TRY(ensure_workspace(ctx, s, kWsMoeAct, static_cast<size_t>(n_tokens * k * inter) * sizeof(float) + 64, &p));
+    OBJ_TRY(ensure_workspace(ctx, s, kWsMoeAct, act_scratch_bytes(n_tokens, k, inter), &p));
     *out = static_cast<float*>(p);
     return 0;
 }
@@ -1002,10 +1014,16 @@ int32_t objeta_hip_moe_layer_shared_device(objeta_hip_context* ctx, int32_t form
     hipStream_t s = resolve_stream(ctx, stream);
     if (n_tokens == 0) return 0;
     if (!d_ids_out || !d_weights_out) OBJ_FAIL(kInvalidInput, "moe_layer_device", "NULL routing output");
-    // a batch whose tokens share experts: each selected expert's matrices once for
-    // all of its tokens
+    // a batch whose tokens share experts: each selected expert's matrices once for all of its
+    // tokens (under capture without that path's workspace, the per-assignment kernels, which a
+    // larger call may have prepared)
     if (out_dim > 0 && d_table && grouped_preferred(format, n_tokens, k, d_shared != nullptr, hidden, intermediate, out_dim) &&
-        grouped_supported(format, n_experts, n_tokens, k, hidden, intermediate, out_dim)) {
+        grouped_supported(format, n_experts, n_tokens, k, hidden, intermediate, out_dim) &&
+        grouped_ready(ctx, s, format, n_experts, n_tokens, k, d_shared != nullptr, hidden, intermediate, out_dim, false)) {
+        // what the batches below kGroupedMinTokens need on the per-assignment kernels
+        const uint64_t few = n_tokens < kGroupedMinTokens ? n_tokens : kGroupedMinTokens - 1;
+        OBJ_TRY(offer_workspace(ctx, s, kWsSelTab, few * k * sizeof(objeta_hip_expert_ptrs)));
+        OBJ_TRY(offer_workspace(ctx, s, kWsMoeAct, act_scratch_bytes(few, k + (d_shared ? 1 : 0), intermediate)));
         OBJ_TRY(launch_router(ctx, s, d_router_w, d_router_bias, d_x, n_tokens, n_experts, hidden, k, renormalize,
                               d_ids_out, d_weights_out, nullptr, nullptr));
         return launch_moe_grouped(ctx, format, s, d_table, n_experts, d_shared, d_ids_out, d_weights_out, n_tokens, k,

@@ -120,6 +120,19 @@ int32_t ensure_workspace(objeta_hip_context* ctx, hipStream_t stream, int slot, 
     return 0;
 }
 
+bool workspace_ready(objeta_hip_context* ctx, hipStream_t stream, int slot, size_t bytes) {
+    for (StreamScratch* sc : ctx->scratch)
+        if (sc->stream == stream && sc->ws[slot].bytes >= bytes) return true;
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    return hipStreamIsCapturing(stream, &st) == hipSuccess && st == hipStreamCaptureStatusNone;
+}
+
+int32_t offer_workspace(objeta_hip_context* ctx, hipStream_t stream, int slot, size_t bytes) {
+    if (!workspace_ready(ctx, stream, slot, bytes)) return 0;
+    void* p = nullptr;
+    return ensure_workspace(ctx, stream, slot, bytes, &p);
+}
+
 int32_t ensure_host_stage(objeta_hip_context* ctx, size_t bytes, void** out) {
     if (ctx->host_stage_bytes < bytes) {
         OBJ_HIP(hipDeviceSynchronize(), "synchronize before staging growth");

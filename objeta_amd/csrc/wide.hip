@@ -66,7 +66,7 @@ struct WideSet {
     uint32_t count, pad[3];
     uint16_t row[32];
 };
-static_assert(sizeof(WideSet) == 128, "one line per set");
+static_assert(sizeof(WideSet) == kWideSetBytes, "one line per set");
 
 // Groups the assignments by expert (workgroup of 256). An assignment's place among its
 // expert's comes from an LDS atomic, so the order inside an expert is not fixed; it
@@ -632,53 +632,12 @@ bool large_work(bool fp4, uint64_t rows, uint64_t cols, uint64_t n_assign, uint6
 
 uint32_t most_sets(uint32_t a, uint32_t n_table, uint32_t members) { return (a < n_table ? a : n_table) + a / members; }
 
-// The workspace of one launch of the layer.
-struct LayerWs {
-    uint32_t* hdr;
-    WideSet *sets, *shared_sets;
-    float *xd, *xmult, *amult, *act, *part;
-    _Float16 *xh, *xl, *ah, *al;
-};
-int32_t layer_workspace(objeta_hip_context* ctx, hipStream_t s, uint64_t T, uint64_t NR, uint32_t n_sets,
-                        uint32_t n_shared, uint64_t H, uint64_t I, uint64_t O, bool official, LayerWs& w) {
-    size_t off = 0;
-    auto take = [&](size_t bytes) {
-        const size_t at = off;
-        off += al256(bytes);
-        return at;
-    };
-    const size_t o_hdr = take(16);
-    const size_t o_set = take(sizeof(WideSet) * ((n_sets + 7) & ~7u));
-    const size_t o_ssh = take(sizeof(WideSet) * ((n_shared + 7) & ~7u));
-    const size_t o_xd = take(official ? 4 * T * H : 0);
-    const size_t o_xm = take(4 * T), o_am = take(4 * NR);
-    const size_t o_xh = take(2 * T * H), o_xl = take(official ? 0 : 2 * T * H);
-    const size_t o_act = take(4 * NR * I), o_ah = take(2 * NR * I), o_al = take(official ? 0 : 2 * NR * I);
-    const size_t o_part = take(4 * NR * O);
-    void* p = nullptr;
-    OBJ_TRY(ensure_workspace(ctx, s, kWsGrouped, off, &p));
-    char* b = static_cast<char*>(p);
-    w.hdr = reinterpret_cast<uint32_t*>(b + o_hdr);
-    w.sets = reinterpret_cast<WideSet*>(b + o_set);
-    w.shared_sets = reinterpret_cast<WideSet*>(b + o_ssh);
-    w.xd = reinterpret_cast<float*>(b + o_xd);
-    w.xmult = reinterpret_cast<float*>(b + o_xm);
-    w.amult = reinterpret_cast<float*>(b + o_am);
-    w.xh = reinterpret_cast<_Float16*>(b + o_xh);
-    w.xl = official ? nullptr : reinterpret_cast<_Float16*>(b + o_xl);
-    w.act = reinterpret_cast<float*>(b + o_act);
-    w.ah = reinterpret_cast<_Float16*>(b + o_ah);
-    w.al = official ? nullptr : reinterpret_cast<_Float16*>(b + o_al);
-    w.part = reinterpret_cast<float*>(b + o_part);
-    return 0;
-}
-
 uint32_t reciprocal(uint64_t k) { return static_cast<uint32_t>(((uint64_t(1) << 20) + k - 1) / k); }
 
-WideArgs gate_up_args(const LayerWs& w, uint32_t hidden, uint32_t inter, uint64_t k, uint32_t a, float limit, bool official) {
+WideArgs gate_up_args(const GroupedWs& w, uint32_t hidden, uint32_t inter, uint64_t k, uint32_t a, float limit, bool official) {
     WideArgs g{};
     g.n = w.hdr;
-    g.sets = w.sets;
+    g.sets = static_cast<WideSet*>(w.sets);
     g.vh = w.xh;
     g.vl = w.xl;
     g.vmult = w.xmult;
@@ -692,10 +651,10 @@ WideArgs gate_up_args(const LayerWs& w, uint32_t hidden, uint32_t inter, uint64_
     return g;
 }
 
-WideArgs down_args(const LayerWs& w, uint32_t inter, uint32_t out_dim, uint32_t a) {
+WideArgs down_args(const GroupedWs& w, uint32_t inter, uint32_t out_dim, uint32_t a) {
     WideArgs g{};
     g.n = w.hdr;
-    g.sets = w.sets;
+    g.sets = static_cast<WideSet*>(w.sets);
     g.vh = w.ah;
     g.vl = w.al;
     g.vmult = w.amult;
@@ -722,8 +681,10 @@ bool matrices_fit(int32_t format, bool official, uint64_t hidden, uint64_t inter
     return below_2g(inter, hidden / 32 * per32) && below_2g(out_dim, inter / 32 * per32);
 }
 
+}  // namespace
+
 // Tokens of one launch: at most kWMaxAssign assignments, split vectors below 2^31 bytes.
-uint64_t launch_tokens(uint64_t k, uint64_t hidden, uint64_t inter) {
+uint64_t wide_tokens(uint64_t k, uint64_t hidden, uint64_t inter) {
     const uint64_t lim = (uint64_t(1) << 31) - 1;
     uint64_t t = kWMaxAssign / k;
     if (t > lim / (2 * hidden)) t = lim / (2 * hidden);
@@ -731,13 +692,11 @@ uint64_t launch_tokens(uint64_t k, uint64_t hidden, uint64_t inter) {
     return t;
 }
 
-}  // namespace
-
 bool wide_supported(int32_t format, uint64_t n_table, uint64_t n_tokens, uint64_t k, uint64_t hidden, uint64_t inter,
                     uint64_t out_dim) {
     if (n_tokens < (format == OBJETA_HIP_FP4_E2M1 ? 1 : kWideMinTokens)) return false;
     return wide_shape(format, n_table, k, hidden, inter, out_dim) && matrices_fit(format, false, hidden, inter, out_dim) &&
-           launch_tokens(k, hidden, inter) > 0;
+           wide_tokens(k, hidden, inter) > 0;
 }
 
 int32_t launch_moe_wide(objeta_hip_context* ctx, int32_t format, hipStream_t s, const objeta_hip_expert_ptrs* table,
@@ -754,20 +713,21 @@ int32_t launch_moe_wide(objeta_hip_context* ctx, int32_t format, hipStream_t s, 
     const bool fp4 = format == OBJETA_HIP_FP4_E2M1, large = large_work(fp4, inter, hidden, n_tokens * k, n_table);
     const uint32_t M = large && !fp4 ? WorkLarge::kMembers : WorkSmall::kMembers;
     // tokens in equal slices (the workspace of a slice is reused by the next)
-    const uint64_t per = launch_tokens(k, hidden, inter), slices = (n_tokens + per - 1) / per;
+    const uint64_t per = wide_tokens(k, hidden, inter), slices = (n_tokens + per - 1) / per;
     const uint64_t slice = (n_tokens + slices - 1) / slices;
     auto sets_of = [&](uint64_t t) {
         return most_sets(static_cast<uint32_t>(t) * kk, E, M) + (shared ? static_cast<uint32_t>((t + M - 1) / M) : 0u);
     };
-    LayerWs w;
-    OBJ_TRY(layer_workspace(ctx, s, slice, slice * k + (shared ? slice : 0), sets_of(slice), 0, hidden, inter, out_dim,
-                            false, w));
+    // the workspace of the longest slice that a smaller batch can have
+    GroupedWs w;
+    OBJ_TRY(grouped_workspace(ctx, s, n_tokens < per ? n_tokens : per, k, n_table, shared != nullptr, hidden, inter, out_dim,
+                              false, w));
     const bool perm = fp4 ? Tile<Fp4Rows>::kPermuted : Tile<QRows<kQ4>>::kPermuted;
     for (uint64_t t0 = 0; t0 < n_tokens; t0 += slice) {
         const uint32_t t = static_cast<uint32_t>(n_tokens - t0 < slice ? n_tokens - t0 : slice), a = t * kk;
         const uint32_t ns = sets_of(t);
         const uint32_t* idt = ids + t0 * k;
-        hipLaunchKernelGGL(wide_prepare_kernel, dim3(1 + t), dim3(256), 0, s, idt, a, E, table, shared, t, M, w.hdr, w.sets,
+        hipLaunchKernelGGL(wide_prepare_kernel, dim3(1 + t), dim3(256), 0, s, idt, a, E, table, shared, t, M, w.hdr, static_cast<WideSet*>(w.sets),
                            static_cast<WideSet*>(nullptr), ctx->err_word, x + t0 * hidden, H, w.xh, w.xl, w.xmult,
                            perm ? 1u : 0u);
         const WideArgs gu = gate_up_args(w, H, I, k, a, limit, false), dn = down_args(w, I, O, a);
@@ -803,7 +763,7 @@ bool official_grouped_supported(uint64_t n_table, uint64_t n_tokens, uint64_t k,
         n_tokens * (k * (matrices / 32 * 17) + matrices) <
             (n_tokens == 2 ? kOfficialGroupedReadBytes2 : kOfficialGroupedReadBytes))
         return false;
-    return matrices_fit(OBJETA_HIP_FP4_E2M1, true, hidden, inter, out_dim) && n_tokens <= launch_tokens(k, hidden, inter);
+    return matrices_fit(OBJETA_HIP_FP4_E2M1, true, hidden, inter, out_dim) && n_tokens <= wide_tokens(k, hidden, inter);
 }
 
 // The official layer of launch_moe_official_fp4 on the grouped products: x is quantized
@@ -832,8 +792,9 @@ int32_t launch_moe_official_grouped(objeta_hip_context* ctx, hipStream_t s, cons
     const uint32_t M = WorkOfficial::kMembers;
     const uint32_t NS = most_sets(A, static_cast<uint32_t>(n_table), M), NSS = shared ? (T + M - 1) / M : 0;
     const uint32_t H = static_cast<uint32_t>(hidden), I = static_cast<uint32_t>(inter), O = static_cast<uint32_t>(out_dim);
-    LayerWs w;
-    OBJ_TRY(layer_workspace(ctx, s, T, NR, NS, NSS, hidden, inter, out_dim, true, w));
+    GroupedWs w;
+    OBJ_TRY(grouped_workspace(ctx, s, T, k, n_table, shared != nullptr, hidden, inter, out_dim, true, w));
+    WideSet* const shared_sets = static_cast<WideSet*>(w.shared_sets);
     auto mark = [&](hipEvent_t e) -> int32_t {
         if (e) OBJ_HIP(hipEventRecord(e, s), "record event");
         return 0;
@@ -842,16 +803,17 @@ int32_t launch_moe_official_grouped(objeta_hip_context* ctx, hipStream_t s, cons
     const uint32_t perm = Tile<Fp4Rows>::kPermuted ? 1u : 0u;
     OBJ_TRY(launch_act_quant(s, x, T, H, nullptr, nullptr, w.xd));
     hipLaunchKernelGGL(wide_prepare_kernel, dim3(1 + T), dim3(256), 0, s, ids, A, static_cast<uint32_t>(n_table), table,
-                       shared, T, M, w.hdr, w.sets, w.shared_sets, ctx->err_word, w.xd, H, w.xh, w.xl, w.xmult, perm);
+                       shared, T, M, w.hdr, static_cast<WideSet*>(w.sets), shared_sets, ctx->err_word, w.xd, H, w.xh,
+                       static_cast<_Float16*>(nullptr), w.xmult, perm);
     const WideArgs gu = gate_up_args(w, H, I, k, A, limit, true), dn = down_args(w, I, O, A);
     auto shared_args = [&](WideArgs g) {
         g.n = w.hdr + 1;
-        g.sets = w.shared_sets;
+        g.sets = shared_sets;
         return g;
     };
     if (shared && !apart) {
-        if (large) launch_wide_pair<WorkOfficial, WorkOfficialSmall, kWGateUp>(s, gu, NS, w.hdr + 1, w.shared_sets, NSS);
-        else launch_wide_pair<WorkOfficialSmall, WorkOfficialSmall, kWGateUp>(s, gu, NS, w.hdr + 1, w.shared_sets, NSS);
+        if (large) launch_wide_pair<WorkOfficial, WorkOfficialSmall, kWGateUp>(s, gu, NS, w.hdr + 1, shared_sets, NSS);
+        else launch_wide_pair<WorkOfficialSmall, WorkOfficialSmall, kWGateUp>(s, gu, NS, w.hdr + 1, shared_sets, NSS);
     } else {
         if (large) launch_wide_phase<Fp4Rows, WorkOfficial, kWGateUp>(s, gu, NS);
         else launch_wide_phase<Fp4Rows, WorkOfficialSmall, kWGateUp>(s, gu, NS);
@@ -862,10 +824,11 @@ int32_t launch_moe_official_grouped(objeta_hip_context* ctx, hipStream_t s, cons
     OBJ_HIP(hipGetLastError(), action);
     OBJ_TRY(launch_act_quant(s, w.act, NR, I, inter_values, inter_scales, w.act));
     OBJ_TRY(mark(marks ? marks->act_quant_end : nullptr));
-    hipLaunchKernelGGL(wide_split_kernel, dim3(NR), dim3(256), 0, s, w.act, I, w.ah, w.al, w.amult, perm);
+    hipLaunchKernelGGL(wide_split_kernel, dim3(NR), dim3(256), 0, s, w.act, I, w.ah, static_cast<_Float16*>(nullptr),
+                       w.amult, perm);
     if (shared && !apart) {
-        if (large) launch_wide_pair<WorkOfficial, WorkOfficialSmall, kWDown>(s, dn, NS, w.hdr + 1, w.shared_sets, NSS);
-        else launch_wide_pair<WorkOfficialSmall, WorkOfficialSmall, kWDown>(s, dn, NS, w.hdr + 1, w.shared_sets, NSS);
+        if (large) launch_wide_pair<WorkOfficial, WorkOfficialSmall, kWDown>(s, dn, NS, w.hdr + 1, shared_sets, NSS);
+        else launch_wide_pair<WorkOfficialSmall, WorkOfficialSmall, kWDown>(s, dn, NS, w.hdr + 1, shared_sets, NSS);
     } else {
         if (large) launch_wide_phase<Fp4Rows, WorkOfficial, kWDown>(s, dn, NS);
         else launch_wide_phase<Fp4Rows, WorkOfficialSmall, kWDown>(s, dn, NS);
@@ -895,28 +858,50 @@ uint32_t gemv_slice(uint32_t batch, uint32_t cols) {
     return ((batch + n - 1) / n + 31) / 32 * 32;
 }
 
+// The GEMV's workspace: the split vectors of a slice, then partial sums. Several ranges are
+// taken only while row blocks x vector groups are below 2 cus, so below 4 cus workgroups in all:
+// a bound that does not fall as the batch grows. At least what gemv_mfma_kernel's passes of
+// 8 vectors take, which a smaller batch may need under capture.
+struct GemvWs {
+    size_t xh, xl, part, bytes;
+};
+template <class K>
+GemvWs gemv_layout(uint32_t cus, uint32_t rows, uint32_t cols, uint32_t batch) {
+    const uint64_t slice = gemv_slice(batch, cols), ks_max = ((cols + 255) / 256 + 1) / 2;
+    const uint64_t tiles = 4ull * cus * K::kMembers * K::kRows, all = ks_max * slice * rows;
+    GemvWs w;
+    w.xh = al256(4 * slice);
+    w.xl = w.xh + al256(2 * slice * cols);
+    w.part = w.xl + al256(2 * slice * cols);
+    w.bytes = w.part + (ks_max > 1 ? al256(4 * (tiles < all ? tiles : all)) : 0);
+    const size_t passes = gemv_passes_bytes(rows, cols, batch);
+    if (w.bytes < passes) w.bytes = passes;
+    return w;
+}
+
+uint32_t cu_count(const objeta_hip_context* ctx) {
+    return ctx->info.compute_units > 0 ? static_cast<uint32_t>(ctx->info.compute_units) : 256u;
+}
+
+// us, large / small work: Q5_0 14336 x 4096 by 32 vectors 37.5 / 41.8, Q4_0 4096 x 4096
+// by 64 25.5 / 24.5, split FP4 5000 x 3584 by 100 36.3 / 34.4
+bool gemv_large(uint64_t rows, uint64_t cols, uint64_t batch) {
+    return batch > WorkSmall::kMembers && rows * cols >= (uint64_t(1) << 25);
+}
+
 template <class R, class K>
 int32_t launch_gemv_wide_t(objeta_hip_context* ctx, hipStream_t s, const void* w, const void* ws, const float* x, float* y,
                            uint32_t rows, uint32_t cols, uint32_t batch) {
-    const uint32_t cus = ctx->info.compute_units > 0 ? static_cast<uint32_t>(ctx->info.compute_units) : 256u;
-    const uint32_t nrb = row_blocks<K, kWGemv>(rows);
-    const uint32_t slice = gemv_slice(batch, cols);
+    const uint32_t cus = cu_count(ctx), nrb = row_blocks<K, kWGemv>(rows), slice = gemv_slice(batch, cols);
     // at most half as many column ranges as the columns have units of 256
     const uint32_t units = (cols + 255) / 256, ks_max = (units + 1) / 2;
-    size_t off = 0;
-    const size_t o_xm = off; off += al256(4ull * slice);
-    const size_t o_xh = off; off += al256(2ull * slice * cols);
-    const size_t o_xl = off; off += al256(2ull * slice * cols);
-    // partial sums: several ranges only while row blocks x vector groups are below 2 cus, so
-    // below 4 cus workgroups in all (a bound that does not fall as the batch grows)
-    const uint64_t tiles = 4ull * cus * K::kMembers * K::kRows, all = static_cast<uint64_t>(ks_max) * slice * rows;
-    const size_t o_part = off; off += ks_max > 1 ? al256(4 * (tiles < all ? tiles : all)) : 0;
+    const GemvWs lay = gemv_layout<K>(cus, rows, cols, batch);
     void* wsp = nullptr;
-    OBJ_TRY(ensure_workspace(ctx, s, kWsGemv, off, &wsp));
+    OBJ_TRY(ensure_workspace(ctx, s, kWsGemv, lay.bytes, &wsp));
     char* b = static_cast<char*>(wsp);
-    float* xmult = reinterpret_cast<float*>(b + o_xm);
-    auto* xh = reinterpret_cast<_Float16*>(b + o_xh);
-    auto* xl = reinterpret_cast<_Float16*>(b + o_xl);
+    float* xmult = reinterpret_cast<float*>(b);
+    auto* xh = reinterpret_cast<_Float16*>(b + lay.xh);
+    auto* xl = reinterpret_cast<_Float16*>(b + lay.xl);
     WideArgs g{};
     g.w0 = w;
     g.s0 = ws;
@@ -934,7 +919,7 @@ int32_t launch_gemv_wide_t(objeta_hip_context* ctx, hipStream_t s, const void* w
         g.range = 256 * ((units + ks - 1) / ks);
         ks = (cols + g.range - 1) / g.range;
         float* const ys = y + static_cast<size_t>(v0) * rows;
-        g.out = ks > 1 ? reinterpret_cast<float*>(b + o_part) : ys;
+        g.out = ks > 1 ? reinterpret_cast<float*>(b + lay.part) : ys;
         g.n_vec = n;
         hipLaunchKernelGGL(wide_split_kernel, dim3(n), dim3(256), 0, s, x + static_cast<size_t>(v0) * cols, cols, xh, xl,
                            xmult, Tile<R>::kPermuted ? 1u : 0u);
@@ -947,12 +932,17 @@ int32_t launch_gemv_wide_t(objeta_hip_context* ctx, hipStream_t s, const void* w
 
 }  // namespace
 
+size_t gemv_wide_bytes(objeta_hip_context* ctx, int32_t format, uint64_t rows, uint64_t cols, uint64_t batch) {
+    const uint32_t R = static_cast<uint32_t>(rows), C = static_cast<uint32_t>(cols), B = static_cast<uint32_t>(batch);
+    const uint32_t cus = cu_count(ctx);
+    if (!gemv_large(rows, cols, batch)) return gemv_layout<WorkSmall>(cus, R, C, B).bytes;
+    return format == OBJETA_HIP_FP4_E2M1 ? gemv_layout<WorkLarge4>(cus, R, C, B).bytes : gemv_layout<WorkLarge>(cus, R, C, B).bytes;
+}
+
 int32_t launch_gemv_wide(objeta_hip_context* ctx, hipStream_t s, int32_t format, const void* w, const void* ws,
                          const float* x, float* y, uint64_t rows, uint64_t cols, uint64_t batch) {
     const uint32_t R = static_cast<uint32_t>(rows), C = static_cast<uint32_t>(cols), B = static_cast<uint32_t>(batch);
-    // us, large / small work: Q5_0 14336 x 4096 by 32 vectors 37.5 / 41.8, Q4_0 4096 x 4096
-    // by 64 25.5 / 24.5, split FP4 5000 x 3584 by 100 36.3 / 34.4
-    const bool large = B > WorkSmall::kMembers && rows * cols >= (uint64_t(1) << 25);
+    const bool large = gemv_large(rows, cols, batch);
 #define OBJ_WIDE(RT, KL)                                                                       \
     (large ? launch_gemv_wide_t<RT, KL>(ctx, s, w, ws, x, y, R, C, B)                          \
            : launch_gemv_wide_t<RT, WorkSmall>(ctx, s, w, ws, x, y, R, C, B))
