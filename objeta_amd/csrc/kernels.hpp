@@ -178,6 +178,10 @@ bool grouped_ready(objeta_hip_context* ctx, hipStream_t s, int32_t format, uint6
                    bool shared, uint64_t hidden, uint64_t inter, uint64_t out_dim, bool official);
 // Tokens of one launch of the wide products.
 uint64_t wide_tokens(uint64_t k, uint64_t hidden, uint64_t inter);
+// Whether a layer of several such launches would write rows of x that a later launch reads:
+// out overlaps x and its rows run ahead of x's (out == x with out_dim <= hidden does not).
+bool wide_overwrites_x(const float* x, const float* out, uint64_t n_tokens, uint64_t k, uint64_t hidden, uint64_t inter,
+                       uint64_t out_dim);
 // Whether the layer entry points run a batch of n_tokens on the grouped path.
 bool grouped_preferred(int32_t format, uint64_t n_tokens, uint64_t k, bool shared, uint64_t hidden, uint64_t inter,
                        uint64_t out_dim);

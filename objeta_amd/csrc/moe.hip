@@ -1019,6 +1019,7 @@ int32_t objeta_hip_moe_layer_shared_device(objeta_hip_context* ctx, int32_t form
     // larger call may have prepared)
     if (out_dim > 0 && d_table && grouped_preferred(format, n_tokens, k, d_shared != nullptr, hidden, intermediate, out_dim) &&
         grouped_supported(format, n_experts, n_tokens, k, hidden, intermediate, out_dim) &&
+        !wide_overwrites_x(d_x, d_out, n_tokens, k, hidden, intermediate, out_dim) &&
         grouped_ready(ctx, s, format, n_experts, n_tokens, k, d_shared != nullptr, hidden, intermediate, out_dim, false)) {
         // what the batches below kGroupedMinTokens need on the per-assignment kernels
         const uint64_t few = n_tokens < kGroupedMinTokens ? n_tokens : kGroupedMinTokens - 1;

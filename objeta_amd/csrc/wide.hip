@@ -692,6 +692,14 @@ uint64_t wide_tokens(uint64_t k, uint64_t hidden, uint64_t inter) {
     return t;
 }
 
+bool wide_overwrites_x(const float* x, const float* out, uint64_t n_tokens, uint64_t k, uint64_t hidden, uint64_t inter,
+                       uint64_t out_dim) {
+    if (n_tokens <= wide_tokens(k, hidden, inter)) return false;
+    const uintptr_t x0 = reinterpret_cast<uintptr_t>(x), o0 = reinterpret_cast<uintptr_t>(out);
+    const bool apart = o0 + 4 * n_tokens * out_dim <= x0 || x0 + 4 * n_tokens * hidden <= o0;
+    return !apart && !(o0 <= x0 && out_dim <= hidden);
+}
+
 bool wide_supported(int32_t format, uint64_t n_table, uint64_t n_tokens, uint64_t k, uint64_t hidden, uint64_t inter,
                     uint64_t out_dim) {
     if (n_tokens < (format == OBJETA_HIP_FP4_E2M1 ? 1 : kWideMinTokens)) return false;

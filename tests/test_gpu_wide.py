@@ -160,6 +160,28 @@ def test_layer_wide(backend, fmt, E, K, T, H, I, shared):
     del keep, keep_s
 
 
+def test_layer_wide_output_over_its_input(backend):
+    """Past one launch's 4096 assignments with outputs that run over the inputs: out == x with
+    wider rows, and with rows as wide, equal the call with buffers of their own."""
+    fmt, E, K, T, H, I = Q4, 8, 8, 600, 64, 64
+    moe = MoeExecutor(backend)
+    d_wr = backend.to_device(orc.gauss(E * H, 5, 0.02))
+    xs = orc.gauss(T * H, 6, 1.0)
+    d_ids, d_w = backend.alloc(4 * T * K), backend.alloc(4 * T * K)
+    for O in (128, 64):
+        experts = make_experts(fmt, E, H, I, O, seed=21, gen="gauss")
+        table, keep = device_table(backend, fmt, experts)
+        d_x, d_out, d_both = backend.to_device(xs), backend.alloc(4 * T * O), backend.alloc(4 * T * O)
+        d_both.upload(np.concatenate([xs, np.zeros(T * (O - H), np.float32)]))
+        for x, out in ((d_x, d_out), (d_both, d_both)):
+            moe.layer_device(fmt, table, d_wr, None, K, T, x, None, out, d_ids, d_w, H, I, O)
+        backend.synchronize()
+        assert moe.device_error() == 0
+        ref = d_out.download(np.float32, T * O)
+        assert float(np.max(np.abs(d_both.download(np.float32, T * O) - ref))) <= 1e-4 * float(np.max(np.abs(ref)))
+        del keep
+
+
 def test_wide_out_of_table_and_repeated_experts(backend):
     fmt, E, K, T, H, I, O = Q4, 4, 2, 40, 256, 128, 264
     experts = make_experts(fmt, E, H, I, O, seed=15, gen="gauss")
