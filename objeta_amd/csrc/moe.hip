@@ -818,13 +818,14 @@ int32_t launch_moe_official_fp4(objeta_hip_context* ctx, hipStream_t s, const ob
         return ((static_cast<size_t>(tokens * hidden) * sizeof(float) + 255) & ~size_t(255)) +
                static_cast<size_t>(tokens * kk * inter) * sizeof(float) + 64;
     };
-    if (official_grouped_supported(n_table, n_tokens, k, hidden, inter, out_dim) &&
+    // (a call that times its phases, marks, has one token)
+    if (!marks && official_grouped_supported(n_table, n_tokens, k, hidden, inter, out_dim) &&
         grouped_ready(ctx, s, OBJETA_HIP_FP4_E2M1, n_table, n_tokens, k, shared != nullptr, hidden, inter, out_dim, true)) {
         // and what the batches below kOfficialGroupedMinTokens need on the per-token kernels
         OBJ_TRY(offer_workspace(ctx, s, kWsOfficial,
                                 per_token_bytes(n_tokens < kOfficialGroupedMinTokens ? n_tokens : kOfficialGroupedMinTokens - 1)));
         return launch_moe_official_grouped(ctx, s, table, n_table, shared, ids, wts, n_tokens, k, x, out, hidden,
-                                           inter, out_dim, limit, inter_values, inter_scales, marks);
+                                           inter, out_dim, limit, inter_values, inter_scales);
     }
     const size_t xb = (static_cast<size_t>(n_tokens * hidden) * sizeof(float) + 255) & ~size_t(255);
     void* ws = nullptr;

@@ -735,12 +735,17 @@ int32_t launch_moe_wide(objeta_hip_context* ctx, int32_t format, hipStream_t s, 
         const uint32_t t = static_cast<uint32_t>(n_tokens - t0 < slice ? n_tokens - t0 : slice), a = t * kk;
         const uint32_t ns = sets_of(t);
         const uint32_t* idt = ids + t0 * k;
-        hipLaunchKernelGGL(wide_prepare_kernel, dim3(1 + t), dim3(256), 0, s, idt, a, E, table, shared, t, M, w.hdr, static_cast<WideSet*>(w.sets),
-                           static_cast<WideSet*>(nullptr), ctx->err_word, x + t0 * hidden, H, w.xh, w.xl, w.xmult,
-                           perm ? 1u : 0u);
+        hipLaunchKernelGGL(wide_prepare_kernel, dim3(1 + t), dim3(256), 0, s, idt, a, E, table, shared, t, M, w.hdr,
+                           static_cast<WideSet*>(w.sets), static_cast<WideSet*>(nullptr), ctx->err_word, x + t0 * hidden, H,
+                           w.xh, w.xl, w.xmult, perm ? 1u : 0u);
         const WideArgs gu = gate_up_args(w, H, I, k, a, limit, false), dn = down_args(w, I, O, a);
         const uint32_t nr = a + (shared ? t : 0);
-#define OBJ_WIDE_LAYER(R, K)                                                                                         {                                                                                                                    launch_wide_phase<R, K, kWGateUp>(s, gu, ns);                                                                    hipLaunchKernelGGL(wide_split_kernel, dim3(nr), dim3(256), 0, s, w.act, I, w.ah, w.al, w.amult,                                    perm ? 1u : 0u);                                                                              launch_wide_phase<R, K, kWDown>(s, dn, ns);                                                                  }
+#define OBJ_WIDE_LAYER(R, K)                                                                                       \
+    {                                                                                                              \
+        launch_wide_phase<R, K, kWGateUp>(s, gu, ns);                                                              \
+        hipLaunchKernelGGL(wide_split_kernel, dim3(nr), dim3(256), 0, s, w.act, I, w.ah, w.al, w.amult, perm ? 1u : 0u); \
+        launch_wide_phase<R, K, kWDown>(s, dn, ns);                                                                \
+    }
         switch (format) {
             case OBJETA_HIP_Q4_0:
                 if (large) OBJ_WIDE_LAYER(QRows<kQ4>, WorkLarge) else OBJ_WIDE_LAYER(QRows<kQ4>, WorkSmall)
@@ -779,14 +784,13 @@ bool official_grouped_supported(uint64_t n_table, uint64_t n_tokens, uint64_t k,
 // their own fp16 high part: what lies below 2^-38 of the row's largest value, past the
 // fp16 subnormals, is dropped, far below the last bit of the fp32 sums), the routed FP4
 // experts and the FP8 shared expert read each matrix once per member set, in one launch
-// per phase unless the caller times them apart (marks), the intermediates are quantized
-// in place, and the combine adds w * down in slot order from zero, then the shared
+// per phase, the intermediates are quantized in place, and the combine adds w * down in slot order from zero, then the shared
 // expert's down.
 int32_t launch_moe_official_grouped(objeta_hip_context* ctx, hipStream_t s, const objeta_hip_expert_ptrs* table,
                                     uint64_t n_table, const objeta_hip_expert_ptrs* shared, const uint32_t* ids,
                                     const float* wts, uint64_t n_tokens, uint64_t k, const float* x, float* out,
                                     uint64_t hidden, uint64_t inter, uint64_t out_dim, float limit,
-                                    uint8_t* inter_values, uint8_t* inter_scales, const OfficialMarks* marks) {
+                                    uint8_t* inter_values, uint8_t* inter_scales) {
     const char* action = "launch official FP4 MoE (grouped)";
     // the routed FP4 and the shared FP8 sets multiply the same split activations
     static_assert(Tile<Fp4Rows>::kPermuted == Tile<Fp8Rows>::kPermuted, "one activation order for both tiles");
@@ -803,45 +807,30 @@ int32_t launch_moe_official_grouped(objeta_hip_context* ctx, hipStream_t s, cons
     GroupedWs w;
     OBJ_TRY(grouped_workspace(ctx, s, T, k, n_table, shared != nullptr, hidden, inter, out_dim, true, w));
     WideSet* const shared_sets = static_cast<WideSet*>(w.shared_sets);
-    auto mark = [&](hipEvent_t e) -> int32_t {
-        if (e) OBJ_HIP(hipEventRecord(e, s), "record event");
-        return 0;
-    };
-    const bool large = large_work(true, inter, hidden, A, n_table), apart = marks != nullptr;
+    const bool large = large_work(true, inter, hidden, A, n_table);
     const uint32_t perm = Tile<Fp4Rows>::kPermuted ? 1u : 0u;
     OBJ_TRY(launch_act_quant(s, x, T, H, nullptr, nullptr, w.xd));
     hipLaunchKernelGGL(wide_prepare_kernel, dim3(1 + T), dim3(256), 0, s, ids, A, static_cast<uint32_t>(n_table), table,
                        shared, T, M, w.hdr, static_cast<WideSet*>(w.sets), shared_sets, ctx->err_word, w.xd, H, w.xh,
                        static_cast<_Float16*>(nullptr), w.xmult, perm);
     const WideArgs gu = gate_up_args(w, H, I, k, A, limit, true), dn = down_args(w, I, O, A);
-    auto shared_args = [&](WideArgs g) {
-        g.n = w.hdr + 1;
-        g.sets = shared_sets;
-        return g;
-    };
-    if (shared && !apart) {
+    if (shared) {
         if (large) launch_wide_pair<WorkOfficial, WorkOfficialSmall, kWGateUp>(s, gu, NS, w.hdr + 1, shared_sets, NSS);
         else launch_wide_pair<WorkOfficialSmall, WorkOfficialSmall, kWGateUp>(s, gu, NS, w.hdr + 1, shared_sets, NSS);
     } else {
         if (large) launch_wide_phase<Fp4Rows, WorkOfficial, kWGateUp>(s, gu, NS);
         else launch_wide_phase<Fp4Rows, WorkOfficialSmall, kWGateUp>(s, gu, NS);
-        OBJ_TRY(mark(marks ? marks->gate_up_end : nullptr));
-        if (shared) launch_wide_phase<Fp8Rows, WorkOfficialSmall, kWGateUp>(s, shared_args(gu), NSS);
-        OBJ_TRY(mark(marks ? marks->shared_gate_up_end : nullptr));
     }
     OBJ_HIP(hipGetLastError(), action);
     OBJ_TRY(launch_act_quant(s, w.act, NR, I, inter_values, inter_scales, w.act));
-    OBJ_TRY(mark(marks ? marks->act_quant_end : nullptr));
     hipLaunchKernelGGL(wide_split_kernel, dim3(NR), dim3(256), 0, s, w.act, I, w.ah, static_cast<_Float16*>(nullptr),
                        w.amult, perm);
-    if (shared && !apart) {
+    if (shared) {
         if (large) launch_wide_pair<WorkOfficial, WorkOfficialSmall, kWDown>(s, dn, NS, w.hdr + 1, shared_sets, NSS);
         else launch_wide_pair<WorkOfficialSmall, WorkOfficialSmall, kWDown>(s, dn, NS, w.hdr + 1, shared_sets, NSS);
     } else {
         if (large) launch_wide_phase<Fp4Rows, WorkOfficial, kWDown>(s, dn, NS);
         else launch_wide_phase<Fp4Rows, WorkOfficialSmall, kWDown>(s, dn, NS);
-        OBJ_TRY(mark(marks ? marks->down_end : nullptr));
-        if (shared) launch_wide_phase<Fp8Rows, WorkOfficialSmall, kWDown>(s, shared_args(dn), NSS);
     }
     launch_moe_combine(s, ids, wts, w.part, shared ? w.part + static_cast<size_t>(A) * O : nullptr, nullptr, out, T,
                        static_cast<uint32_t>(k), O, static_cast<uint32_t>(n_table));
