@@ -703,6 +703,8 @@ bool wide_overwrites_x(const float* x, const float* out, uint64_t n_tokens, uint
 bool wide_supported(int32_t format, uint64_t n_table, uint64_t n_tokens, uint64_t k, uint64_t hidden, uint64_t inter,
                     uint64_t out_dim) {
     if (n_tokens < (format == OBJETA_HIP_FP4_E2M1 ? 1 : kWideMinTokens)) return false;
+    // refused by every form, as by the per-assignment kernels
+    if (n_tokens > 0x7FFFFFFFull || n_tokens * k * inter > 0x7FFFFFFFull || n_tokens * out_dim > 0x7FFFFFFFull) return false;
     return wide_shape(format, n_table, k, hidden, inter, out_dim) && matrices_fit(format, false, hidden, inter, out_dim) &&
            wide_tokens(k, hidden, inter) > 0;
 }

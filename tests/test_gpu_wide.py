@@ -9,7 +9,7 @@ import numpy as np
 import pytest
 import torch
 
-from objeta_amd import HipBackend, MoeExecutor, QGemvShape, QuantBackend, QuantFormat
+from objeta_amd import ExpertTable, HipBackend, HipError, MoeExecutor, QGemvShape, QuantBackend, QuantFormat
 from objeta_amd.api import check
 from oracle import oracle as orc
 from test_gpu_grouped import skewed_selection
@@ -180,6 +180,23 @@ def test_layer_wide_output_over_its_input(backend):
         ref = d_out.download(np.float32, T * O)
         assert float(np.max(np.abs(d_both.download(np.float32, T * O) - ref))) <= 1e-4 * float(np.max(np.abs(ref)))
         del keep
+
+
+def test_layer_past_the_index_range_is_refused():
+    """tokens * k * intermediate above 2^31: InvalidInput, whichever kernels a layer's batch
+    takes."""
+    be = HipBackend(0, 1)
+    E, K, T, H, I = 32, 32, 4096, 64, 16448
+    one = make_experts(Q4, 1, H, I, H, seed=2, gen="gauss")
+    _, keep = device_table(be, Q4, one)
+    table = ExpertTable(be, [tuple(keep)] * E)
+    d_x, d_wr = be.to_device(orc.gauss(T * H, 1, 1.0)), be.to_device(orc.gauss(E * H, 2, 0.02))
+    d_out, d_ids, d_w = be.alloc(4 * T * H), be.alloc(4 * T * K), be.alloc(4 * T * K)
+    with pytest.raises(HipError) as e:
+        MoeExecutor(be).layer_device(Q4, table, d_wr, None, K, T, d_x, None, d_out, d_ids, d_w, H, I, H)
+    assert e.value.kind == "InvalidInput"
+    be.synchronize()
+    be.close()
 
 
 def test_wide_out_of_table_and_repeated_experts(backend):
