@@ -911,7 +911,7 @@ bool grouped_supported(int32_t format, uint64_t n_table, uint64_t n_tokens, uint
         out_dim > (1u << 20))
         return false;
     // split FP4 runs on the sets of eight for few assignments alone, which are wide_supported
-    return format != OBJETA_HIP_FP4_E2M1;
+    return format != OBJETA_HIP_FP4_E2M1 && matrices_fit(format, false, hidden, inter, out_dim);
 }
 
 namespace {
@@ -1008,7 +1008,7 @@ int32_t launch_moe_grouped(objeta_hip_context* ctx, int32_t format, hipStream_t 
         OBJ_FAIL(kUnsupported, action, "hidden and intermediate must be non-zero multiples of 64 (<= 2^20)");
     if (format == OBJETA_HIP_FP4_E2M1 && (hidden % 128 || inter % 128))
         OBJ_FAIL(kUnsupported, action, "the grouped path takes split-FP4 experts with hidden and intermediate % 128 == 0");
-    if (format == OBJETA_HIP_FP4_E2M1 && !few) OBJ_FAIL(kUnsupported, action, "split-FP4 matrices above 2^31 bytes");
+    if (!matrices_fit(format, false, hidden, inter, out_dim)) OBJ_FAIL(kUnsupported, action, "matrices above 2^31 bytes");
     if (!table || !ids || !wts || !x || !out) OBJ_FAIL(kInvalidInput, action, "NULL device pointer");
     if (reinterpret_cast<uintptr_t>(x) % 16) OBJ_FAIL(kInvalidInput, action, "x must be 16-byte aligned");
     const uint32_t A = static_cast<uint32_t>(n_tokens * k), T = static_cast<uint32_t>(n_tokens);

@@ -176,6 +176,9 @@ int32_t grouped_workspace(objeta_hip_context* ctx, hipStream_t s, uint64_t n_tok
 // Whether launch_moe_grouped (launch_moe_official_grouped) has its workspace or may make it.
 bool grouped_ready(objeta_hip_context* ctx, hipStream_t s, int32_t format, uint64_t n_table, uint64_t n_tokens, uint64_t k,
                    bool shared, uint64_t hidden, uint64_t inter, uint64_t out_dim, bool official);
+// Whether an expert's matrices lie below 2^31 bytes, as every grouped form's 32-bit offsets need
+// (`official`: with an FP8 shared expert's).
+bool matrices_fit(int32_t format, bool official, uint64_t hidden, uint64_t inter, uint64_t out_dim);
 // Tokens of one launch of the wide products.
 uint64_t wide_tokens(uint64_t k, uint64_t hidden, uint64_t inter);
 // Whether a layer of several such launches would write rows of x that a later launch reads:

@@ -674,14 +674,14 @@ bool wide_shape(int32_t format, uint64_t n_table, uint64_t k, uint64_t hidden, u
     return format != OBJETA_HIP_FP4_E2M1 || (hidden % 128 == 0 && inter % 128 == 0);
 }
 
-// Matrices of at most 2^31 bytes (FP8, the widest of the formats, when `official`).
+}  // namespace
+
+// FP8 is the widest of the formats.
 bool matrices_fit(int32_t format, bool official, uint64_t hidden, uint64_t inter, uint64_t out_dim) {
     const uint64_t per32 = official ? 32 : format == OBJETA_HIP_Q4_0 ? 18 : format == OBJETA_HIP_Q5_0 ? 22
                          : format == OBJETA_HIP_IQ3_0 ? 14 : 16;
     return below_2g(inter, hidden / 32 * per32) && below_2g(out_dim, inter / 32 * per32);
 }
-
-}  // namespace
 
 // Tokens of one launch: at most kWMaxAssign assignments, split vectors below 2^31 bytes.
 uint64_t wide_tokens(uint64_t k, uint64_t hidden, uint64_t inter) {

@@ -291,6 +291,39 @@ def test_layer_sets_of_eight_with_shared_expert(backend, fmt, E, K, T, H, I):
     test_layer_batch_runs_grouped_with_shared_expert(backend, fmt, E, K, T, H, I, 0.0)
 
 
+def test_layer_of_matrices_above_2g(backend):
+    """A down matrix of 2.2 GB (3700 rows of 2^20 columns, rows past 2^31 bytes among them): the
+    grouped products' 32-bit offsets do not reach it, so the layer runs on the per-assignment
+    kernels and the direct grouped call refuses it."""
+    import torch
+    T, H, I, O = 12, 64, 1 << 20, 3700
+    row = I // 32 * 18
+    experts = make_experts(Q4, 1, H, I, 1, seed=4, gen="gauss")
+    up = [backend.to_device(m[0]) for m in experts[0][:2]]
+    down = torch.randint(0, 256, (O, I // 32, 18), dtype=torch.uint8, device="cuda")
+    down[:, :, 0:2] = torch.tensor([0x00, 0x18], dtype=torch.uint8, device="cuda")  # scale 2^-9
+    torch.cuda.synchronize()
+    assert down.numel() > 1 << 31
+    table = ExpertTable(backend, [(up[0], up[1], down.data_ptr())])
+    xs = orc.gauss(T * H, 5, 1.0)
+    d_x, d_wr = backend.to_device(xs), backend.to_device(orc.gauss(H, 6, 0.02))
+    d_out, d_ids, d_w = backend.alloc(4 * T * O), backend.alloc(4 * T), backend.alloc(4 * T)
+    moe = MoeExecutor(backend)
+    moe.layer_device(Q4, table, d_wr, None, 1, T, d_x, None, d_out, d_ids, d_w, H, I, O)
+    with pytest.raises(HipError) as e:
+        moe.grouped_device(Q4, table, d_ids, d_w, T, 1, d_x, None, d_out, H, I, O)
+    assert e.value.kind == "Unsupported"
+    backend.synchronize()
+    out = d_out.download(np.float32, T * O).reshape(T, O)
+    last = O - 1
+    assert last * row > 1 << 31
+    sample = [0, 1700, last - 1, last]
+    mats = down[sample].cpu().numpy().reshape(-1)
+    for t in (0, T - 1):
+        ref = orc.selected_moe(Q4, [(experts[0][0][0], experts[0][1][0], mats)], [(0, 1.0)], xs[t * H:(t + 1) * H], H, I, 4)
+        assert float(np.max(np.abs(out[t, sample] - ref))) <= 1e-4 * float(np.max(np.abs(ref)))
+
+
 @pytest.mark.parametrize("fmt,K,T,H,I,shared,grouped", [
     (Q4, 8, 4, 4096, 768, False, False),   # 162 MiB of assigned experts
     (Q4, 8, 7, 4096, 768, False, True),    # 284
