@@ -349,6 +349,7 @@ def test_official_layer_batch_grouped(backend, T, k, with_shared):
     (14, 1, 4736, 1152, False),
     (14, 1, 4096, 1536, True),   # whole chunks; the shared expert in two sets, the second of six
     (6, 4, 7168, 1408, True),    # past the few: the wide products' 128-row work with a short chunk
+    (6, 4, 7168, 1408, False),
 ])
 def test_official_layer_few_assignments_on_large_matrices(backend, T, k, hidden, inter, with_shared):
     """At most 14 assignments of top-1 or top-2 on large matrices: sets of eight, the FP8
@@ -360,6 +361,21 @@ def test_official_layer_few_assignments_on_large_matrices(backend, T, k, hidden,
     selections = [[(int(e), float(w)) for e, w in zip(rng.choice(n, k, replace=False),
                                                       rng.dirichlet(np.ones(k)).astype(F32))] for _ in range(T)]
     xs = orc.gauss(T * hidden, 92 + T, 2.0).reshape(T, hidden)
+    out, q, s = run_official(backend, experts, shared, selections, xs, hidden, inter, out_dim)
+    check_official(out, q, s, experts, shared, selections, xs, hidden, inter, out_dim)
+
+
+@pytest.mark.parametrize("T", [257, 300, 1030])
+def test_official_layer_many_assignments(backend, T):
+    """Four slots: 1028 and 1200 assignments on the grouped products (17 and 19 sets of the
+    shared expert), 4120 on the per-token kernels."""
+    hidden, inter, out_dim, n, k = 256, 128, 256, 6, 4
+    experts = [fp4_random_expert(hidden, inter, out_dim, 600 + 3 * e) for e in range(n)]
+    shared = fp8_random_expert(hidden, inter, out_dim, 79)
+    rng = np.random.default_rng(T)
+    selections = [[(int(e), float(w)) for e, w in zip(rng.choice(n, k, replace=False),
+                                                      rng.dirichlet(np.ones(k)).astype(F32))] for _ in range(T)]
+    xs = orc.gauss(T * hidden, 93 + T, 2.0).reshape(T, hidden)
     out, q, s = run_official(backend, experts, shared, selections, xs, hidden, inter, out_dim)
     check_official(out, q, s, experts, shared, selections, xs, hidden, inter, out_dim)
 

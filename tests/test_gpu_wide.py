@@ -1,5 +1,6 @@
 """Products with many vectors (wide.hip) on the GPU: the batched GEMV from 9 vectors and
-the experts of a layer from 9 tokens, against the CPU oracle. Work items hold 16 vectors and
+the experts of a layer from 9 tokens (with more than 72 assignments; split FP4 and IQ3_0 40),
+against the CPU oracle. Work items hold 16 vectors and
 workgroups 64 weight rows (32 of gate and of up) in 256-column chunks; for large matrices
 with many vectors 32 (split FP4: 16), 128 and 128 (256); launches take 4096 assignments. The
 sizes lie at the edges of these."""
@@ -77,7 +78,11 @@ def test_gemv_wide_large_matrix(backend, fmt, cols):
         _assert_close(y[t], orc.gemv(int(fmt), q, xt, rows, cols), q, xt, fmt, rows, cols)
 
 
-@pytest.mark.parametrize("rows,cols,batch", [(5, 128, 9), (128, 256, 16), (300, 1152, 33)])
+@pytest.mark.parametrize("rows,cols,batch", [
+    (5, 128, 9), (128, 256, 16), (300, 1152, 33),
+    (8260, 4096, 17), (8260, 4096, 33),  # the large work: a second and a third work item of one vector
+    (8260, 4224, 33),                    # with a short last chunk
+])
 def test_fp4_split_gemv_wide(backend, rows, cols, batch):
     rng = np.random.default_rng(rows + cols)
     w = rng.integers(0, 256, size=rows * cols // 2, dtype=np.uint8)
@@ -118,36 +123,41 @@ def test_gemv_wide_non_finite_and_extreme_vectors(backend):
 
 
 @pytest.mark.parametrize("fmt,E,K,T,H,I,shared", [
-    (Q4, 16, 4, 9, 256, 128, False),      # the smallest batch
+    (Q4, 16, 4, 9, 256, 128, False),      # few assignments: sets of eight in the direct call
+    (Q4, 16, 9, 9, 256, 128, False),      # the smallest batch of 9 tokens that is not few
     (Q5, 3, 2, 33, 192, 64, True),        # short chunks, inter of one row block
     (IQ3, 7, 3, 70, 320, 192, True),
     (FP4, 5, 4, 65, 256, 384, True),
     (Q4, 6, 4, 1030, 64, 64, True),       # two launches' worth of assignments
-    (Q4, 2, 2, 33, 1024, 1024, False),    # the large work: two vector tiles, and one over
+    (Q4, 2, 2, 33, 1024, 1024, False),    # few assignments again: 66
+    (Q4, 2, 2, 65, 1024, 1024, False),    # the large work: two vector tiles, twice, and one over
+    (Q4, 2, 2, 37, 1024, 1024, False),    # 74
     (Q5, 2, 1, 47, 1088, 1024, True),     # with a short chunk
     (IQ3, 2, 2, 70, 1024, 1088, False),   # with ragged row blocks
     (FP4, 2, 2, 40, 1152, 1024, True),
 ])
 def test_layer_wide(backend, fmt, E, K, T, H, I, shared):
-    """objeta_hip_moe_layer_shared_device at batches: the oracle's routing and
-    selected_moe for tokens across the batch, and the per-assignment path for all."""
+    """objeta_hip_moe_layer_shared_device at batches, and the direct grouped call on its
+    selection where that takes it: the oracle's routing and selected_moe for tokens across
+    the batch, and the per-assignment path for all."""
     experts = make_experts(fmt, E + 1, H, I, H, seed=140 + fmt, gen="gauss")
     table, keep = device_table(backend, fmt, experts[:E])
     sh, keep_s = device_table(backend, fmt, experts[E:]) if shared else (None, None)
     w_r = orc.gauss(E * H, 150 + fmt, 0.02)
     xs = orc.gauss(T * H, 160 + fmt, 1.0).reshape(T, H)
     d_x = backend.to_device(xs.ravel())
-    d_out, d_ref = backend.alloc(4 * T * H), backend.alloc(4 * T * H)
+    d_out, d_ref, d_grp = (backend.alloc(4 * T * H) for _ in range(3))
     d_ids, d_w = backend.alloc(4 * T * K), backend.alloc(4 * T * K)
     moe = MoeExecutor(backend)
     moe.layer_device(fmt, table, backend.to_device(w_r), None, K, T, d_x, d_x, d_out, d_ids, d_w, H, I, H, shared=sh)
-    if not shared and T * K <= 1024:  # the layer groups from 12 tokens on
-        moe.grouped_device(fmt, table, d_ids, d_w, T, K, d_x, d_x, d_out, H, I, H)
+    direct = not shared and T * K <= 1024
+    if direct:
+        moe.grouped_device(fmt, table, d_ids, d_w, T, K, d_x, d_x, d_grp, H, I, H)
     moe.selected_device(fmt, table, d_ids, d_w, T, K, d_x, d_x, d_ref, H, I, H, shared=sh)
     backend.synchronize()
     assert moe.device_error() == 0
     ids = d_ids.download(np.uint32, T * K).reshape(T, K)
-    out = d_out.download(np.float32, T * H).reshape(T, H)
+    outs = [b.download(np.float32, T * H).reshape(T, H) for b in ([d_out, d_grp] if direct else [d_out])]
     per = d_ref.download(np.float32, T * H).reshape(T, H)
     oe = oracle_experts(fmt, experts)
     for t in {0, 1, T // 3, T // 2, T // 2 + 1, T - 1}:
@@ -155,8 +165,10 @@ def test_layer_wide(backend, fmt, E, K, T, H, I, shared):
         assert np.array_equal(ids[t], rid), t
         sel = [(int(i), float(v)) for i, v in zip(rid, rw)]
         ref = orc.selected_moe(fmt, oe[:E], sel, xs[t], H, I, H, shared=oe[E] if shared else None)
-        assert_moe_close(out[t] - xs[t], ref)
-    assert float(np.max(np.abs(out - per))) <= 1e-4 * float(np.max(np.abs(per)))
+        for out in outs:
+            assert_moe_close(out[t] - xs[t], ref)
+    for out in outs:
+        assert float(np.max(np.abs(out - per))) <= 1e-4 * float(np.max(np.abs(per)))
     del keep, keep_s
 
 
