@@ -316,7 +316,8 @@ int32_t objeta_hip_moe_selected_device_noalloc(objeta_hip_context* ctx, int32_t 
  * result (within the fp32 tolerance) as objeta_hip_moe_selected_device; no
  * reference counterpart as one call (execute_selected_moe_cuda, moe.rs:352-751,
  * runs each selected expert per token). Limits: n_experts <= 1024, n_tokens * k
- * <= 1024, hidden and intermediate multiples of 64; Unsupported outside them.
+ * <= 1024, hidden and intermediate multiples of 64, matrices below 2^31 bytes;
+ * Unsupported outside them.
  * d_ids is required. An out-of-table id sets bit 1 of the device error word and
  * makes that token's output NaN. Non-finite block scales give a non-finite output
  * element, but not necessarily the same special value as the reference's
@@ -344,12 +345,16 @@ int32_t objeta_hip_moe_down_device(objeta_hip_context* ctx, int32_t format, obje
  * d_router_w [n_experts][hidden] (+ d_router_bias) writes d_ids_out/d_weights_out
  * [n_tokens][k], then the selected experts of d_table (n_experts entries) run:
  * below 12 tokens on the per-assignment kernels of objeta_hip_moe_selected_device,
- * from 12 tokens on the grouped-token products of objeta_hip_moe_grouped_device (any
- * number of tokens) whenever that path takes the shape; from 2 tokens when one expert's
- * three matrices take 8 MiB or more, or n_tokens * k experts' 128 MiB or more (what the
- * per-assignment kernels would read). The two agree within the fp32
- * tolerance, not bit for bit. No host
- * synchronisation; graph-capturable. No reference counterpart as one call: the
+ * from 12 tokens on the grouped-token products of objeta_hip_moe_grouped_device (without
+ * that call's limit of 1024 assignments) whenever that path takes the shape; from 2 tokens
+ * when one expert's three matrices take 8 MiB or more, or n_tokens * k experts' 128 MiB or
+ * more (what the per-assignment kernels would read; 168 to 256 MiB, or not below 12 tokens
+ * at all, where hidden is 2048, 4096 or a larger power of two and the intermediate at most
+ * 1024). The two agree within the fp32 tolerance, not bit for bit. At most 4096 tokens (the
+ * router's limit). d_out may be d_residual or d_x. No host synchronisation; graph-capturable
+ * (after an eager call of as many tokens on the stream, which makes the workspaces; a
+ * captured call without the grouped products' runs on the per-assignment kernels if theirs
+ * are there). No reference counterpart as one call: the
  * reference routes on the host (deepseek_single_layer_moe.rs:687-743) and then
  * calls execute_selected_moe_cuda. */
 int32_t objeta_hip_moe_layer_device(objeta_hip_context* ctx, int32_t format, objeta_hip_stream stream,
@@ -569,10 +574,11 @@ int32_t objeta_hip_fp8_act_fp8_weight_gemv_device(objeta_hip_context* ctx, objet
  * d_inter_scales [n_tokens*kk][intermediate/128] (nullable; kk = k + 1 with a
  * shared expert, else k) receive the intermediates' FP8 codes: rows t*k + j for
  * the routed slots, then n_tokens*k + t for the shared expert. From 6 tokens
- * (2 where the per-token kernels would read 256 MiB or more of expert weights; up to 4096
- * (token, slot) assignments over at most 1024 experts) the layer runs on the
- * grouped-token products of objeta_hip_moe_grouped_device: each selected expert, and the
- * shared expert, read once per set of up to 16 of its tokens. The
+ * (3 where the per-token kernels would read 256 MiB or more of expert weights, 2 from 288
+ * MiB; up to 4096 (token, slot) assignments over at most 1024 experts) the layer runs on
+ * the grouped-token products of objeta_hip_moe_grouped_device: each selected expert, and
+ * the shared expert, read once per set of up to 16 of its tokens (8 at top-1 and top-2
+ * with at most 14 assignments of large matrices). The
  * results agree with the per-token kernels within the fp32 tolerance (the sums run
  * in another order), so an intermediate code near a rounding boundary can differ. */
 int32_t objeta_hip_moe_official_fp4_device(objeta_hip_context* ctx, objeta_hip_stream stream,

@@ -987,8 +987,8 @@ bool grouped_preferred(int32_t format, uint64_t n_tokens, uint64_t k, bool share
 }
 
 int32_t launch_moe_grouped(objeta_hip_context* ctx, int32_t format, hipStream_t s, const objeta_hip_expert_ptrs* table,
-                           uint64_t n_table, const objeta_hip_expert_ptrs* shared, const uint32_t* ids, const float* wts, uint64_t n_tokens, uint64_t k,
-                           const float* x, const float* resid, float* out, uint64_t hidden, uint64_t inter,
+                           uint64_t n_table, const objeta_hip_expert_ptrs* shared, const uint32_t* ids, const float* wts,
+                           uint64_t n_tokens, uint64_t k, const float* x, const float* resid, float* out, uint64_t hidden, uint64_t inter,
                            uint64_t out_dim, float limit) {
     const char* action = "launch grouped-token MoE";
     if (format < OBJETA_HIP_Q4_0 || format > OBJETA_HIP_FP4_E2M1)

@@ -138,10 +138,12 @@ int32_t launch_gemv_mfma(objeta_hip_context* ctx, hipStream_t s, int32_t format,
 // tokens 73.3 / 72.0, 16 tokens 85.1 / 76.4, 32 tokens 146.8 / 104.4).
 constexpr uint64_t kGroupedMinTokens = 12;
 // From 2 tokens when one expert's three matrices take at least this many bytes: at
-// hidden 7168 / intermediate 2048 (23 MB FP4 experts, a shared expert) the grouped
-// path takes 160 / 258 / 314 us at 2 / 3 / 4 tokens against 218 / 360 / 459 on the
-// per-assignment kernels; the Qwen3-A3B shape's 2.6 MB experts keep the 12-token
-// switch.
+// hidden 7168 / intermediate 2048 (23 MB FP4 experts, a shared expert, top-8) the grouped
+// path takes 123 / 165 / 185 us at 2 / 3 / 4 tokens against 214 / 313 / 406 on the
+// per-assignment kernels, top-2 65 / 73 / 81 against 72 / 99 / 130. Only at 2 to 4
+// assignments in all are the per-assignment kernels ahead (top-1 without a shared expert
+// 42 / 52 / 62 against 50 / 57 / 59). The Qwen3-A3B shape's 2.6 MB experts keep the
+// 12-token switch.
 constexpr uint64_t kGroupedLargeExpertBytes = uint64_t(8) << 20;
 // And from 2 tokens when the per-assignment kernels would read this many bytes (us,
 // per-assignment / grouped: Q5_0 2048 x 1408 top-4 at 6 tokens, 136 MiB, 63 / 46; Q4_0 2560
@@ -192,9 +194,9 @@ bool grouped_preferred(int32_t format, uint64_t n_tokens, uint64_t k, bool share
 bool grouped_supported(int32_t format, uint64_t n_table, uint64_t n_tokens, uint64_t k, uint64_t hidden,
                        uint64_t inter, uint64_t out_dim);
 int32_t launch_moe_grouped(objeta_hip_context* ctx, int32_t format, hipStream_t s, const objeta_hip_expert_ptrs* table,
-                           uint64_t n_table, const objeta_hip_expert_ptrs* shared, const uint32_t* ids, const float* wts, uint64_t n_tokens, uint64_t k,
-                           const float* x, const float* resid, float* out, uint64_t hidden, uint64_t inter,
-                           uint64_t out_dim, float limit);
+                           uint64_t n_table, const objeta_hip_expert_ptrs* shared, const uint32_t* ids, const float* wts,
+                           uint64_t n_tokens, uint64_t k, const float* x, const float* resid, float* out,
+                           uint64_t hidden, uint64_t inter, uint64_t out_dim, float limit);
 
 // Whether launch_moe_grouped takes the sets of eight for the batch where the wide products
 // take it too (measured at the definition).

@@ -772,7 +772,7 @@ int32_t launch_moe_selected(objeta_hip_context* ctx, int32_t format, hipStream_t
 
 // ------------------------------------------------------- official FP4 layer
 // execute_selected_moe_official_routed_fp4_cuda (moe.rs:1393-1663) for a batch of
-// tokens (from kOfficialGroupedMinTokens tokens on, launch_moe_official_grouped), in
+// tokens (where official_grouped_supported, launch_moe_official_grouped), in
 // six launches: act_quant(x) dequantized; the routed gate/up (FP4 split
 // weights, official SwiGLU) of every (token, slot); the shared expert's gate/up
 // (FP8 weights) into the rows after them; act_quant of all intermediates,

@@ -68,8 +68,9 @@ OBJ_HD float div_rn(float a, float b) {
 // Dev. 34, 1990), three operations instead of a division's ten. Divisors outside
 // [2^-96, 2^96] (where a product could leave the normal range; |a / b| <= 16 here, and a
 // quotient small enough to underflow rounds to the zero point either way) are divided.
-// 4096 x 14336 on the device, us: Q4_0 72 -> 41, Q5_0 312 -> 46, IQ3_0 134 -> 39 (with the
-// rounding below eight operations less and the bit fields gathered in registers).
+// 4096 x 14336 on the device, us, the same input again (part of it cached): Q4_0 72 -> 41, Q5_0
+// 312 -> 46, IQ3_0 134 -> 39, with the rounding below eight operations less and the bit
+// fields gathered in registers; new inputs each time: Q4_0 67 -> 51, the memory's rate.
 struct Quotient {
     float b, r;
     bool divide;

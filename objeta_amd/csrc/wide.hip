@@ -16,12 +16,13 @@
 // What bounds it: with few vectors per expert the weights' loads in flight (3.1 to 3.4
 // TB/s); with many, latency and the LDS reads. At 512 tokens of hidden 2048, intermediate
 // 768, 128 experts, top-8 (Q4_0) the matrix cores are about a quarter busy and the VALU a
-// third. Layer times there by shape (vectors, rows, columns of a chunk; workgroups per CU):
+// third. Layer times there by shape (vectors, rows, columns of a chunk; workgroups per CU),
+// all on one input whose router selection alone takes 78 us:
 // 64, 128, 128; 2: 476 us. 32, 128, 128; 3: 353 (in 128 registers, 100 bytes of spills: 663).
 // 32, 64, 256; 4: 440. 32, 64, 128; 5: 570. 32, 256, 128; 2: 419. 32, 128, 256; 2: 388. 16, 64,
-// 256; 4: 376. Before: the per-assignment kernels 1893 us; sets of eight 188 us for the
-// 97-token Q5_0 layer that takes 123 here; eight passes of gemv_mfma_kernel 73 us for 64
-// vectors by 4096 x 4096 (Q4_0; 24.6 here).
+// 256; 4: 376. Over inputs in turn, before and now: that layer 1844 -> 311 us (the
+// per-assignment kernels), a 97-token Q5_0 layer 195 -> 133 (sets of eight), 64 vectors by
+// 4096 x 4096 (Q4_0) 74 -> 25 (eight passes of gemv_mfma_kernel).
 //
 // Rounding (relative to 64-bit results, against the kernels before): a running sum over
 // 256 columns (split FP4: 512), added to a total, keeps the chains short. The two parts'
@@ -619,12 +620,14 @@ bool below_2g(uint64_t rows, uint64_t bytes_per_row) { return rows * bytes_per_r
 
 // Large work (128 weight rows per workgroup) where the matrices are large and an expert
 // has many vectors; 64 rows otherwise (more workgroups, a shorter chain of chunks each).
-// us per layer, large / small: Q4_0 2048 x 768, 128 experts, top-8 at 512 tokens 366 /
-// 376, at 200 181 / 178; Q4_0 4096 x 1536, 64 experts at 256 tokens 505 / 543, at 40 280 /
-// 233; IQ3_0 2048 x 2048 at 300 tokens 443 / 520; Q4_0 1024 x 512, 16 experts at 250 tokens
-// 63 / 59. Split FP4 work items hold 16 vectors in both: from about one vector per expert
-// of very large matrices (7168 x 2048, 64 experts, 32 tokens 411 / 435; official, 256
-// experts, 6 tokens 195 / 187).
+// us per layer, large / small, each pair on one input: Q4_0 2048 x 768, 128 experts, top-8 at
+// 512 tokens 366 / 376, at 200 181 / 178; Q4_0 4096 x 1536, 64 experts at 256 tokens 505 /
+// 543, at 40 280 / 233; IQ3_0 2048 x 2048 at 300 tokens 443 / 520; Q4_0 1024 x 512, 16
+// experts at 250 tokens 63 / 59. The assignments are the whole call's, not one launch's
+// slice of them: 384 experts at 1000 tokens of Q5_0 2048 x 768, top-8, in two launches 904 /
+// 932. Split FP4 work items hold 16 vectors in both: from about one vector per expert of
+// very large matrices (7168 x 2048, 64 experts, 32 tokens 411 / 435; official, 256 experts,
+// 6 tokens 195 / 187).
 bool large_work(bool fp4, uint64_t rows, uint64_t cols, uint64_t n_assign, uint64_t n_table) {
     return (n_assign >= 16 * n_table && rows * cols >= (uint64_t(1) << 20)) ||
            (fp4 && n_assign >= n_table && rows * cols >= (uint64_t(8) << 20));
